@@ -158,10 +158,10 @@ static bool verbose() {
   return e && *e && *e != '0';
 }
 
-// Tuned two-pass schedule per (sector shape, precision); the chain shapes
-// (the ch_* fields) also on their own, for pinned operator schedules.
-static std::map<std::tuple<int, int, int, int, int>, TwoPassCfg>& tp_cache() {
-  static std::map<std::tuple<int, int, int, int, int>, TwoPassCfg> m;
+// Tuned operator schedule per (sector shape, column stride, precision), and
+// the chain shapes (the ch_* fields) per (sector shape, precision).
+static std::map<std::tuple<int, int, int, int, int, int>, TwoPassCfg>& tp_cache() {
+  static std::map<std::tuple<int, int, int, int, int, int>, TwoPassCfg> m;
   return m;
 }
 static std::map<std::tuple<int, int, int, int, int>, TwoPassCfg>& tp_chain_cache() {
@@ -201,16 +201,10 @@ static std::vector<int> dw_chunk_counts(int dimdw, int slots, bool with32 = true
   return v;
 }
 
-// Pick panel widths, block sizes and grids of the two passes by timing the
-// operator on the sector itself (3 launches per candidate after a warm-up).
+// EDL_TWO_PASS_CFG_F32 / _F64, parsed and checked: whether the environment
+// pins the operator schedule of this precision.
 template <typename T>
-static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s) {
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, (int)sizeof(T));
-  // timed on the engine's own (padded) layout
-  const int ld = padded_ld(s.sp[0].dim);
-  const TwoPassView V = two_pass_view(s, ld);
-  TwoPassCfg best;
-  bool pinned = false;
+static bool two_pass_pin(const TwoPassView& V, TwoPassCfg& best) {
   // EDL_TWO_PASS_CFG_F32 / _F64 =
   // "C,threads_up,grid_up,R,threads_dw,nchunk[,ncol,kch[,up_rpt,up_kch[,dw_vec[,up_col[,dw_rng[,dw_ord]]]]]]"
   // pins the operator schedule of that precision (reproducible profiles of
@@ -255,42 +249,48 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s) {
               "EDL_TWO_PASS_CFG_F32/_F64: bad block size, grid or chunk count");
     EDL_CHECK(256 * sizeof(T) + 16 + (size_t)V.dimup * p.C * sizeof(T) <= (size_t)(160 * 1024),
               "EDL_TWO_PASS_CFG_F32/_F64: up-pass columns exceed LDS");
-    pinned = true;
     best = p;
-  } else {
-    auto it = tp_cache().find(key);
-    if (it != tp_cache().end()) return it->second;
+    return true;
   }
-  // The chain shapes do not depend on the operator's: a pinned operator
-  // schedule still runs its chains on their own tuned shapes.
-  auto ct = tp_chain_cache().find(key);
-  // A pinned range-blocked down pass (dw_rng > 0) or one in the locality
-  // order of columns (dw_ord = 1) pins the chain's down pass to the same
-  // form, so that its Lanczos terms are tested pinned too.
-  auto pin_chain_range = [&](TwoPassCfg& b) {
-    if (!pinned || (b.dw_rng == 0 && b.dw_ord == 0)) return;
-    b.ch_R = b.R;
-    b.ch_threads = b.threads_dw;
-    b.ch_nchunk = b.nchunk;
-    b.ch_ncol = b.ncol;
-    b.ch_kch = b.kch;
-    b.ch_vec = b.dw_rng > 0 ? 0 : b.dw_vec;
-    b.ch_rng = b.dw_rng;
-    b.ch_ord = b.dw_ord;
-  };
-  if (pinned && ct != tp_chain_cache().end()) {
-    with_chain_shapes(best, ct->second);
-    pin_chain_range(best);
-    return best;
-  }
+  return false;
+}
+
+// Pick panel widths, block sizes and grids of the two passes by timing the
+// operator on the sector itself, in the layout it will run on (ld): a first
+// launch of each candidate, and three more where that one was not slower
+// than twice the best so far.
+template <typename T>
+static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s, int ld) {
+  const TwoPassView V = two_pass_view(s, ld);
+  TwoPassCfg best;
+  if (two_pass_pin<T>(V, best)) return best;
+  // (layouts of different strides tune apart: the down pass prefers other
+  // shapes where its row segments straddle cache lines)
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, ld, (int)sizeof(T));
+  auto it = tp_cache().find(key);
+  if (it != tp_cache().end()) return it->second;
   hipStream_t st = c.stream;
   const int64_t D = s.dim, Dp = (int64_t)ld * s.sp[1].dim;
-  DevBuf d64(sizeof(double) * D), q(sizeof(T) * Dp), t(sizeof(T) * Dp), o(sizeof(T) * Dp);
-  launch_start_vector(d64.as<double>(), D, 0x5EEDull, st);
-  launch_zero_bytes(q.p, sizeof(T) * Dp, st);
-  launch_convert_ld<T>(d64.as<double>(), q.as<T>(), s.sp[0].dim, s.sp[1].dim, ld, st);
+  DevBuf q(sizeof(T) * Dp), t(sizeof(T) * Dp), o(sizeof(T) * Dp);
+  {
+    DevBuf d64(sizeof(double) * D);
+    launch_start_vector(d64.as<double>(), D, 0x5EEDull, st);
+    launch_zero_bytes(q.p, sizeof(T) * Dp, st);
+    launch_convert_ld<T>(d64.as<double>(), q.as<T>(), s.sp[0].dim, s.sp[1].dim, ld, st);
+    EDL_HIP(hipStreamSynchronize(st));
+  }
   const int lds = 160 * 1024;
-  if (!pinned) {
+  // mean ms of one launch
+  auto timed = [&](const std::function<void()>& launch, double best_ms) {
+    EventTimer first(st);
+    launch();
+    const double one = first.stop();
+    if (one > 2.0 * best_ms) return one;
+    EventTimer tm(st);
+    for (int r = 0; r < 3; ++r) launch();
+    return tm.stop() / 3;
+  };
+  {
     best.grid_up = c.num_cu;
     best.nchunk = std::min(32, V.dimdw);
     double best_up = 1e300, best_dw = 1e300;
@@ -311,14 +311,12 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s) {
           w.up_kch = rk % 100;
           w.threads_up = th;
           w.grid_up = c.num_cu * gm;
-          launch_pass_up<T>(V, c.model.inter, lut_dev<T>(s.sp[0]), q.as<T>(), q.as<T>(), t.as<T>(), nullptr, w, st);
-          EventTimer tm(st);
-          for (int r = 0; r < 3; ++r)
+          const double ms = timed([&]() {
             launch_pass_up<T>(V, c.model.inter, lut_dev<T>(s.sp[0]), q.as<T>(), q.as<T>(), t.as<T>(), nullptr, w, st);
-          const double ms = tm.stop();
+          }, best_up);
           if (verbose())
             std::fprintf(stderr, "[edl] tune up  fp%d C %d col %d rpt %d kch %2d threads %4d grid %5d: %.4f ms\n",
-                         8 * (int)sizeof(T), C, col, w.up_rpt, w.up_kch, th, w.grid_up, ms / 3);
+                         8 * (int)sizeof(T), C, col, w.up_rpt, w.up_kch, th, w.grid_up, ms);
           if (ms < best_up) {
             best_up = ms;
             best.C = C;
@@ -350,14 +348,12 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s) {
           w.dw_vec = vo >= 1;
           w.dw_ord = vo == 2;
           if (pass_dw_lds_bytes(V, w) > (size_t)lds - 4096) continue;
-          launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), q.as<T>(), q.as<T>(), t.as<T>(), o.as<T>(), nullptr, w, st);
-          EventTimer tm(st);
-          for (int r = 0; r < 3; ++r)
+          const double ms = timed([&]() {
             launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), q.as<T>(), q.as<T>(), t.as<T>(), o.as<T>(), nullptr, w, st);
-          const double ms = tm.stop();
+          }, best_dw);
           if (verbose())
             std::fprintf(stderr, "[edl] tune dw  fp%d vec %d ord %d R %3d ncol %d kch %2d threads %4d chunks %3d: %.4f ms\n",
-                         8 * (int)sizeof(T), w.dw_vec, w.dw_ord, R, nc, kc, th, nch, ms / 3);
+                         8 * (int)sizeof(T), w.dw_vec, w.dw_ord, R, nc, kc, th, nch, ms);
           if (ms < best_dw) {
             best_dw = ms;
             best.R = R;
@@ -379,14 +375,12 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s) {
           w.R = R;
           w.threads_dw = th;
           w.dw_rng = b;
-          launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), q.as<T>(), q.as<T>(), t.as<T>(), o.as<T>(), nullptr, w, st);
-          EventTimer tm(st);
-          for (int r = 0; r < 3; ++r)
+          const double ms = timed([&]() {
             launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), q.as<T>(), q.as<T>(), t.as<T>(), o.as<T>(), nullptr, w, st);
-          const double ms = tm.stop();
+          }, best_dw);
           if (verbose())
             std::fprintf(stderr, "[edl] tune dw  fp%d ranges b %d (%d) R %3d threads %4d: %.4f ms\n",
-                         8 * (int)sizeof(T), b, V.rng_n[b], R, th, ms / 3);
+                         8 * (int)sizeof(T), b, V.rng_n[b], R, th, ms);
           if (ms < best_dw) {
             best_dw = ms;
             best.R = R;
@@ -396,6 +390,47 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s) {
           }
         }
   }
+  tp_cache()[key] = best;
+  return best;
+}
+
+// The shapes a Lanczos chain's two passes run (the ch_* fields), timed on the
+// engine's own (padded) layout, once per sector shape; they do not depend on
+// the operator's, which a pin may set (with_chain_shapes).
+template <typename T>
+static TwoPassCfg two_pass_chain_cfg(Ctx& c, const Sector& s) {
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, (int)sizeof(T));
+  const int ld = padded_ld(s.sp[0].dim);
+  const TwoPassView V = two_pass_view(s, ld);
+  TwoPassCfg best;
+  const bool pinned = two_pass_pin<T>(V, best);
+  // A pinned range-blocked down pass (dw_rng > 0) or one in the locality
+  // order of columns (dw_ord = 1) pins the chain's down pass to the same
+  // form, so that its Lanczos terms are tested pinned too.
+  auto pin_chain_range = [&](TwoPassCfg& b) {
+    if (!pinned || (b.dw_rng == 0 && b.dw_ord == 0)) return;
+    b.ch_R = b.R;
+    b.ch_threads = b.threads_dw;
+    b.ch_nchunk = b.nchunk;
+    b.ch_ncol = b.ncol;
+    b.ch_kch = b.kch;
+    b.ch_vec = b.dw_rng > 0 ? 0 : b.dw_vec;
+    b.ch_rng = b.dw_rng;
+    b.ch_ord = b.dw_ord;
+  };
+  auto ct = tp_chain_cache().find(key);
+  if (ct != tp_chain_cache().end()) {
+    with_chain_shapes(best, ct->second);
+    pin_chain_range(best);
+    return best;
+  }
+  hipStream_t st = c.stream;
+  const int64_t D = s.dim, Dp = (int64_t)ld * s.sp[1].dim;
+  DevBuf d64(sizeof(double) * D), q(sizeof(T) * Dp), t(sizeof(T) * Dp), o(sizeof(T) * Dp);
+  launch_start_vector(d64.as<double>(), D, 0x5EEDull, st);
+  launch_zero_bytes(q.p, sizeof(T) * Dp, st);
+  launch_convert_ld<T>(d64.as<double>(), q.as<T>(), s.sp[0].dim, s.sp[1].dim, ld, st);
+  const int lds = 160 * 1024;
   // The chain step's down pass (MODE 1) streams two more vectors and holds
   // more registers; its best vector-gather shape is timed on its own, with
   // the chain scalars in a middle-step state that repeated launches leave
@@ -538,7 +573,6 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s) {
           }
   }
   tp_chain_cache()[key] = best;
-  if (!pinned) tp_cache()[key] = best;
   pin_chain_range(best);
   return best;
 }
@@ -575,16 +609,15 @@ static int seg_cols_pin() {
 }
 
 template <typename T>
-static TwoPassCfg seg_cfg(Ctx& c, Sector& s) {
-  static std::map<std::tuple<int, int, int, int, int, int, int, int>, TwoPassCfg> cache;
+static TwoPassCfg seg_cfg(Ctx& c, Sector& s, int ld) {
+  static std::map<std::tuple<int, int, int, int, int, int, int, int, int>, TwoPassCfg> cache;
   const int pin = (seg_rank_pin() == 1 && !seg_rank_ok(s)) ? 0 : seg_rank_pin();
   const int cpin = seg_cols_pin();
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, (int)sizeof(T),
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, ld, (int)sizeof(T),
                                    seg_row_cap(sizeof(T), 1), pin, cpin);
   auto it = cache.find(key);
   if (it != cache.end()) return it->second;
   hipStream_t st = c.stream;
-  const int ld = padded_ld(s.sp[0].dim);
   const TwoPassView V = two_pass_view(s, ld);
   const size_t bytes = sizeof(T) * (size_t)ld * s.sp[1].dim;
   DevBuf v(bytes), t(bytes), o(bytes);
@@ -658,8 +691,9 @@ static TwoPassCfg seg_cfg(Ctx& c, Sector& s) {
   }
   // The chain step's down pass (MODE 1) over a few vector-gather shapes,
   // with the chain scalars in a middle-step state that repeated launches
-  // leave unchanged (beta = 0, norms 1), as for two-pass sectors.
-  {
+  // leave unchanged (beta = 0, norms 1), as for two-pass sectors (chains run
+  // on the engine's padded layout only).
+  if (ld == padded_ld(s.sp[0].dim)) {
     LzScalars s0{};
     s0.s_cur = 1.0;
     s0.s_old = 1.0;
@@ -734,7 +768,7 @@ template <typename T>
 static void apply_h(Ctx& c, Sector& s, const T* v, T* out, int ld, hipStream_t st) {
   if (seg_path(s, sizeof(T))) {
     // columns larger than LDS: segmented up pass, then the down pass
-    const TwoPassCfg cfg = seg_cfg<T>(c, s);
+    const TwoPassCfg cfg = seg_cfg<T>(c, s, ld);
     seg_bounds(s, sizeof(T), cfg.C);
     T* tmp = static_cast<T*>(scratch(c, sizeof(T) * (size_t)ld * s.sp[1].dim));
     const TwoPassView V = two_pass_view(s, ld);
@@ -743,7 +777,7 @@ static void apply_h(Ctx& c, Sector& s, const T* v, T* out, int ld, hipStream_t s
     launch_nonlocal<T>(V, c.model.inter, vin, vin, tmp, nullptr, st);
     launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), vin, vin, tmp, out, nullptr, cfg, st);
   } else if (two_pass_ok(s, sizeof(T))) {
-    const TwoPassCfg cfg = two_pass_cfg<T>(c, s);
+    const TwoPassCfg cfg = two_pass_cfg<T>(c, s, ld);
     T* tmp = static_cast<T*>(scratch(c, sizeof(T) * (size_t)ld * s.sp[1].dim));
     const TwoPassView V = two_pass_view(s, ld);
     T* vin = const_cast<T*>(v);  // operator mode only reads it
@@ -1185,7 +1219,7 @@ static GsRun gs_run(Ctx& c, Sector& S, const double* d_start, int niter, double 
   // Two-pass chains keep their vectors with the padded column stride.
   const int ld = two ? padded_ld(S.sp[0].dim) : S.sp[0].dim;
   if (two) {
-    tps.cfg = chain_cfg(seg ? seg_cfg<T>(c, S) : two_pass_cfg<T>(c, S));
+    tps.cfg = chain_cfg(seg ? seg_cfg<T>(c, S, ld) : two_pass_chain_cfg<T>(c, S));
     if (seg) {
       seg_bounds(S, sizeof(T), tps.cfg.C);
       tps.seg = &S;
@@ -1586,7 +1620,7 @@ static void hxv_noalloc_impl(Ctx& c, Sector& s, const T* v, T* hv) {
   EDL_CHECK(bytes <= noalloc_scratch_bytes(),
             "edl_hxv_noalloc: the sector's intermediate (" + std::to_string(bytes) +
                 " bytes) exceeds the 256 MiB scratch; use edl_hxv");
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, (int)sizeof(T));
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, ld, (int)sizeof(T));
   TwoPassCfg cfg;
   auto it = tp_cache().find(key);
   if (it != tp_cache().end()) {
@@ -2281,7 +2315,7 @@ static int64_t tridiag_group(Ctx& c, const std::vector<SeedSpec>& seeds, const s
       Sector& J = get_sector(c, targets[idx[k]]);
       const bool seg = seg_path(J, sizeof(T));
       TwoPassStep<T> tps{};
-      tps.cfg = chain_cfg(seg ? seg_cfg<T>(c, J) : two_pass_cfg<T>(c, J));
+      tps.cfg = chain_cfg(seg ? seg_cfg<T>(c, J, chains[k].ld) : two_pass_chain_cfg<T>(c, J));
       if (seg) {
         seg_bounds(J, sizeof(T), tps.cfg.C);
         tps.seg = &J;
@@ -2530,7 +2564,7 @@ static void bench_passes_impl(Ctx& c, Sector& s, int reps, double* ms_pass, int3
   for (auto& e : ev) EDL_HIP(hipEventCreate(&e));
   TwoPassCfg cf{};
   if (seg) {
-    cf = seg_cfg<T>(c, s);
+    cf = seg_cfg<T>(c, s, ld);
     seg_bounds(s, sizeof(T), cf.C);
     const TwoPassView V = two_pass_view(s, ld);
     T* tmp = static_cast<T*>(scratch(c, sizeof(T) * (size_t)Dp));
@@ -2544,7 +2578,7 @@ static void bench_passes_impl(Ctx& c, Sector& s, int reps, double* ms_pass, int3
       EDL_HIP(hipEventRecord(ev[3 * r + 2], st));
     }
   } else if (two) {
-    cf = two_pass_cfg<T>(c, s);
+    cf = two_pass_cfg<T>(c, s, ld);
     const TwoPassView V = two_pass_view(s, ld);
     T* tmp = static_cast<T*>(scratch(c, sizeof(T) * (size_t)Dp));
     for (int r = 0; r < reps; ++r) {

@@ -616,28 +616,46 @@ __global__ __launch_bounds__(1024) void k_pass_dw(TwoPassView V, const T* __rest
   }
 }
 
-// Vector-gather down pass (R-row panels, R = 16 to 128, 256 in fp32; padded
-// layout: ld % 32 == 0).  A lane loads VW = 16 / sizeof(T) consecutive rows
-// with one 16-byte load, so an R-row neighbour segment takes LPS = R / VW
-// lanes and one wave instruction fetches GPW = 64 / LPS segments: lane group
-// g takes the hops k = g, g + GPW, g + 2 GPW, ... of the wave's column, and
-// the groups' sums meet by lane shuffles.  Against one 4-byte element per
-// lane this issues GPW times fewer gather instructions for the same bytes,
-// and it admits panels taller than a wave (longer neighbour segments, the
-// shape that ran fastest).  Same block mapping, modes and LDS column table
-// as k_pass_dw.  A quad that straddles DimUp loads rows of the column's
-// padding (inside the column) and stores only rows < DimUp.  With V.ord_dw
-// set, chunk positions are taken in the locality order: position k is
-// column ord_dw[k] (staged in LDS with the chunk's words, which come from the
-// reordered table), so the columns a panel's concurrent blocks work on
-// gather from a narrower window of the panel.
+template <typename T>
+struct Row16;  // 16 bytes of consecutive rows: in registers / LDS, and at element alignment in memory
+template <>
+struct Row16<float> {
+  typedef float type __attribute__((ext_vector_type(4)));
+  typedef float mem __attribute__((ext_vector_type(4), aligned(4)));
+};
+template <>
+struct Row16<double> {
+  typedef double type __attribute__((ext_vector_type(2)));
+  typedef double mem __attribute__((ext_vector_type(2), aligned(8)));
+};
+
+// Vector-gather down pass (R-row panels, R = 16 to 128, 256 in fp32).  A lane
+// loads VW = 16 / sizeof(T) consecutive rows with one 16-byte load, so an R-row
+// neighbour segment takes LPS = R / VW lanes and one wave instruction fetches
+// GPW = 64 / LPS segments: lane group g takes the hops k = g, g + GPW, g + 2
+// GPW, ... of the wave's column, and the groups' sums meet by lane shuffles.
+// Against one 4-byte element per lane this issues GPW times fewer gather
+// instructions for the same bytes, and it admits panels taller than a wave
+// (longer neighbour segments, the shape that ran fastest).  Same block mapping,
+// modes and LDS column table as k_pass_dw.  Any column stride of at least VW
+// rows and any alignment of the elements (Row16::mem): a caller's vectors in
+// the natural layout too, whose row segments straddle one cache line more (4x4,
+// (8,8), DimUp 12 870: edl_hxv 1.94 -> 1.40 ms in fp32, 3.96 -> 2.91 ms in fp64
+// against the one-element form those calls ran before; 3x6, (9,9), fp32 27.9 ->
+// 21.6 ms). The last lane of a column takes the column's last VW rows and
+// stores only those the lane before it does not.  With V.ord_dw set, chunk
+// positions are taken in the locality order: position k is column ord_dw[k]
+// (staged in LDS with the chunk's words, which come from the reordered table),
+// so the columns a panel's concurrent blocks work on gather from a narrower
+// window of the panel.
 template <typename T, int R, int MODE, int NCOL, int KCH>
 __global__ __launch_bounds__(1024) void k_pass_dwv(TwoPassView V, const T* __restrict__ lut_dw, T* qa, T* qb,
                                                    const T* __restrict__ tin, T* outp, LzChain A, int nchunk) {
   constexpr int VW = 16 / (int)sizeof(T);
   constexpr int LPS = R / VW;
   constexpr int GPW = 64 / LPS;
-  typedef T VT __attribute__((ext_vector_type(VW)));
+  typedef typename Row16<T>::type VT;
+  typedef typename Row16<T>::mem VM;
   __shared__ T lut[256];
   __shared__ double sh[16];
   LzScalars s{};
@@ -683,10 +701,12 @@ __global__ __launch_bounds__(1024) void k_pass_dwv(TwoPassView V, const T* __res
   const T bo = (MODE == 1) ? (T)(s.beta_k / s.s_old) : (T)0;
   double part = 0.0;
   if (p < npan) {
-    const int iup0 = p * R + l * VW;
-    const bool ok = iup0 < dimup;
-    const int iuc = ok ? iup0 : 0;
-    const int nval = ok ? min(VW, dimup - iup0) : 0;  // rows of the quad below DimUp
+    const int rw = p * R + l * VW;  // the lane's first own row
+    const bool ok = rw < dimup;
+    const int iuc = ok ? max(min(rw, dimup - VW), 0) : 0;  // its first row read
+    const int own = ok ? rw - iuc : 0;                     // leading rows that belong to the lane before
+    const int end = min(VW, dimup - iuc);                  // (VW, less in columns of fewer rows)
+    const bool full = own == 0 && end == VW;
     const bool lead = ok && g == 0;
     for (int c0 = cb + wave; c0 < ce; c0 += NCOL * nwaves) {
       int col[NCOL], nh[NCOL], cx[NCOL];
@@ -703,9 +723,9 @@ __global__ __launch_bounds__(1024) void k_pass_dwv(TwoPassView V, const T* __res
         nmax = nh[h] > nmax ? nh[h] : nmax;
         const size_t i = (size_t)cx[h] * ld + iuc;
         const bool live = lead && okc[h];
-        t0[h] = live ? __builtin_nontemporal_load(reinterpret_cast<const VT*>(&tin[i])) : (VT)0;
-        o0[h] = (MODE == 1 && live) ? __builtin_nontemporal_load(reinterpret_cast<const VT*>(&out[i])) : (VT)0;
-        q0v[h] = (MODE == 1 && live) ? *reinterpret_cast<const VT*>(&q[i]) : (VT)0;
+        t0[h] = live ? (VT)__builtin_nontemporal_load(reinterpret_cast<const VM*>(&tin[i])) : (VT)0;
+        o0[h] = (MODE == 1 && live) ? (VT)__builtin_nontemporal_load(reinterpret_cast<const VM*>(&out[i])) : (VT)0;
+        q0v[h] = (MODE == 1 && live) ? (VT)*reinterpret_cast<const VM*>(&q[i]) : (VT)0;
         acc[h] = (VT)0;
       }
       for (int k0 = 0; k0 < nmax; k0 += GPW * KCH) {
@@ -725,7 +745,7 @@ __global__ __launch_bounds__(1024) void k_pass_dwv(TwoPassView V, const T* __res
 #pragma unroll
           for (int j = 0; j < KCH; ++j) {
             const uint32_t nbr = w[h][j] & 0xFFFFFFu;
-            x[h][j] = (k0 + g + GPW * j < nh[h]) ? *reinterpret_cast<const VT*>(&q[(size_t)nbr * ld + iuc]) : (VT)0;
+            x[h][j] = (k0 + g + GPW * j < nh[h]) ? (VT)*reinterpret_cast<const VM*>(&q[(size_t)nbr * ld + iuc]) : (VT)0;
           }
 #pragma unroll
         for (int h = 0; h < NCOL; ++h)
@@ -745,22 +765,22 @@ __global__ __launch_bounds__(1024) void k_pass_dwv(TwoPassView V, const T* __res
 #pragma unroll
         for (int h = 0; h < NCOL; ++h) {
           if (!okc[h]) continue;
-          const size_t i = (size_t)cx[h] * ld + iup0;
+          const size_t i = (size_t)cx[h] * ld + iuc;
           VT tv;
           if (MODE == 0) {
             tv = t0[h] + acc[h];
           } else {
             tv = (t0[h] + acc[h]) * ts - bo * o0[h];
           }
-          if (nval == VW) {
-            __builtin_nontemporal_store(tv, reinterpret_cast<VT*>(&out[i]));
+          if (full) {
+            __builtin_nontemporal_store(tv, reinterpret_cast<VM*>(&out[i]));
             if (MODE == 1)
 #pragma unroll
               for (int e = 0; e < VW; ++e) part += (double)tv[e] * (double)q0v[h][e];
           } else {
 #pragma unroll
             for (int e = 0; e < VW; ++e)
-              if (e < nval) {
+              if (e >= own && e < end) {
                 out[i + e] = tv[e];
                 if (MODE == 1) part += (double)tv[e] * (double)q0v[h][e];
               }
@@ -1726,9 +1746,9 @@ static void launch_dwv_n(const TwoPassView& V, const T* lut, T* qa, T* qb, const
 
 bool pass_dw_vec_ok(const TwoPassView& V, const TwoPassCfg& cfg, size_t elem, const void* const* bufs, int nbufs) {
   const bool rok = cfg.R == 16 || cfg.R == 32 || cfg.R == 64 || cfg.R == 128 || (cfg.R == 256 && elem == 4);
-  if (!cfg.dw_vec || !rok || V.ld % 32 != 0) return false;
+  if (!cfg.dw_vec || !rok || V.ld < (int)(16 / elem)) return false;
   for (int i = 0; i < nbufs; ++i)
-    if (bufs[i] && reinterpret_cast<uintptr_t>(bufs[i]) % 16 != 0) return false;
+    if (bufs[i] && reinterpret_cast<uintptr_t>(bufs[i]) % elem != 0) return false;
   return true;
 }
 
@@ -1754,9 +1774,9 @@ static void launch_dw_r(const TwoPassView& V, const T* lut, T* qa, T* qb, const 
   }
   const void* bufs[4] = {qa, qb, tin, out};
   if (cfg.dw_vec && !pass_dw_vec_ok(V, cfg, sizeof(T), bufs, 4)) {
-    // natural layout (ld = DimUp) or unaligned caller buffers: the 4-byte form
+    // a column stride below the rows a lane takes: the one-element form
     // (operator mode only: a chain's partial count follows its own form)
-    EDL_CHECK(MODE == 0, "launch_pass_dw: the chain step's vector-gather down pass needs the padded, aligned layout");
+    EDL_CHECK(MODE == 0, "launch_pass_dw: the chain step's vector-gather down pass needs the padded layout");
     cfg.dw_vec = 0;
     cfg.ncol = 2;
     cfg.kch = 8;

@@ -151,7 +151,7 @@ bool pass_dwr_ok(const TwoPassView& V, int R, int b, size_t elem);
 // LzChain::part_dw; blocks of an up-pass launch, the size of part_up.
 int pass_dw_grid(const TwoPassView& V, const TwoPassCfg& cfg);
 // Whether a launch with this schedule runs the vector-gather down pass
-// (padded layout and 16-byte aligned buffers; otherwise the 4-byte form).
+// (a column stride of 16 bytes or more; otherwise one element a lane).
 bool pass_dw_vec_ok(const TwoPassView& V, const TwoPassCfg& cfg, size_t elem, const void* const* bufs, int nbufs);
 // Dynamic LDS of a down-pass block (column table and offsets).
 size_t pass_dw_lds_bytes(const TwoPassView& V, const TwoPassCfg& cfg);
