@@ -158,6 +158,12 @@ static bool verbose() {
   return e && *e && *e != '0';
 }
 
+// What a spin's hop tables let a schedule choose: their width, and whether the
+// two-hop forms exist (one hopping magnitude).  Part of every schedule key:
+// sectors of one shape on lattices of one and of several hopping values share
+// no schedule.
+static int hop_key(const SpinTable& t) { return 2 * t.kmax + (t.nvals == 1 ? 1 : 0); }
+
 // Tuned operator schedule per (sector shape, column stride, precision), and
 // the chain shapes (the ch_* fields) per (sector shape, precision).
 static std::map<std::tuple<int, int, int, int, int, int>, TwoPassCfg>& tp_cache() {
@@ -266,7 +272,7 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s, int ld) {
   if (two_pass_pin<T>(V, best)) return best;
   // (layouts of different strides tune apart: the down pass prefers other
   // shapes where its row segments straddle cache lines)
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, ld, (int)sizeof(T));
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s.sp[0]), hop_key(s.sp[1]), ld, (int)sizeof(T));
   auto it = tp_cache().find(key);
   if (it != tp_cache().end()) return it->second;
   hipStream_t st = c.stream;
@@ -399,7 +405,7 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s, int ld) {
 // the operator's, which a pin may set (with_chain_shapes).
 template <typename T>
 static TwoPassCfg two_pass_chain_cfg(Ctx& c, const Sector& s) {
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, (int)sizeof(T));
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s.sp[0]), hop_key(s.sp[1]), (int)sizeof(T));
   const int ld = padded_ld(s.sp[0].dim);
   const TwoPassView V = two_pass_view(s, ld);
   TwoPassCfg best;
@@ -613,8 +619,8 @@ static TwoPassCfg seg_cfg(Ctx& c, Sector& s, int ld) {
   static std::map<std::tuple<int, int, int, int, int, int, int, int, int>, TwoPassCfg> cache;
   const int pin = (seg_rank_pin() == 1 && !seg_rank_ok(s)) ? 0 : seg_rank_pin();
   const int cpin = seg_cols_pin();
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, ld, (int)sizeof(T),
-                                   seg_row_cap(sizeof(T), 1), pin, cpin);
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s.sp[0]), hop_key(s.sp[1]), ld, (int)sizeof(T),
+                                   seg_row_cap(sizeof(T), 1), 2 * pin + (seg_rank_ok(s) ? 1 : 0), cpin);
   auto it = cache.find(key);
   if (it != cache.end()) return it->second;
   hipStream_t st = c.stream;
@@ -1620,7 +1626,7 @@ static void hxv_noalloc_impl(Ctx& c, Sector& s, const T* v, T* hv) {
   EDL_CHECK(bytes <= noalloc_scratch_bytes(),
             "edl_hxv_noalloc: the sector's intermediate (" + std::to_string(bytes) +
                 " bytes) exceeds the 256 MiB scratch; use edl_hxv");
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, s.sp[0].kmax, s.sp[1].kmax, ld, (int)sizeof(T));
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s.sp[0]), hop_key(s.sp[1]), ld, (int)sizeof(T));
   TwoPassCfg cfg;
   auto it = tp_cache().find(key);
   if (it != tp_cache().end()) {
@@ -1974,7 +1980,9 @@ static std::vector<BtChain> bt_resized(std::vector<BtChain> v, const BtShape& s)
 template <typename T>
 static BtShape bt_tune(Ctx& c, const std::vector<BtChain>& chains, int max_up, int max_dw, hipStream_t st) {
   const char* fk = std::getenv("EDL_BATCHED_UP_H16");
-  const auto key = std::make_tuple((int)sizeof(T), max_up, max_dw, (int)chains.size(), fk ? std::atoi(fk) : -1);
+  const int forms = (bt_h16_ok(chains, 0) ? 1 : 0) + (bt_h16_ok(chains, 1) ? 2 : 0);  // two-hop tables of each spin
+  const auto key = std::make_tuple((int)sizeof(T), max_up, max_dw, (int)chains.size(),
+                                   4 * (fk ? std::atoi(fk) + 1 : 0) + forms);
   auto it = bt_cache().find(key);
   if (it != bt_cache().end()) return it->second;
   BtShape best = bt_shape(max_up, max_dw, sizeof(T));
