@@ -14,6 +14,7 @@
 #include "batched2.hpp"
 #include "chains.hpp"
 #include "hxv2.hpp"
+#include "resident.hpp"
 #include "seeds.hpp"
 #include "tridiag.hpp"
 
@@ -1206,6 +1207,129 @@ struct GsRun {
   int64_t hxv = 0;
 };
 
+// Small sectors (res_ok) run their chains resident, a chain to a block, unless
+// a pinned schedule or a forced segmentation asks for the two-pass step.
+static bool resident_sector(const Sector& S, size_t elem) {
+  return !std::getenv("EDL_UP_SEGMENT_ROWS") && !std::getenv("EDL_TWO_PASS_CFG_F32") &&
+         !std::getenv("EDL_TWO_PASS_CFG_F64") && res_ok(S, elem);
+}
+
+// The chain of a resident launch on sector S without its start and outputs.
+template <typename T>
+static ResChain res_chain(const Sector& S, int nmax) {
+  ResChain r{};
+  r.V = two_pass_view(S, S.sp[0].dim);
+  r.lut_up = lut_dev<T>(S.sp[0]);
+  r.lut_dw = lut_dev<T>(S.sp[1]);
+  r.nmax = nmax;
+  r.brk_tol = 1e-14;
+  return r;
+}
+static bool res_one(const Sector& S) { return S.sp[0].nvals <= 1 && S.sp[1].nvals <= 1; }
+
+// Scalars and coefficients of one chain as a resident launch leaves them:
+// {LzScalars, alpha[nmax], beta[nmax]}, one device-to-host copy.
+static size_t res_out_bytes(int nmax) { return sizeof(LzScalars) + 2 * sizeof(double) * (size_t)nmax; }
+static ChainOut res_out(const char* p, int nmax) {
+  ChainOut o;
+  LzScalars sc;
+  std::memcpy(&sc, p, sizeof(sc));
+  const double* a = reinterpret_cast<const double*>(p + sizeof(sc));
+  o.nsteps = sc.nsteps;
+  o.norm2 = sc.norm2;
+  o.alpha.assign(a, a + nmax);
+  o.beta.assign(a + nmax, a + 2 * nmax);
+  return o;
+}
+
+// gs_run on a small sector: the whole chain (or `check` steps of it at a time
+// where a tolerance may end it) in one launch, its vectors stored as they are
+// made; EDL_LANCZOS_BASIS=0, or no memory for them, takes a second launch that
+// adds up the eigenvector instead.
+template <typename T>
+static GsRun gs_run_resident(Ctx& c, Sector& S, const double* d_start, int nmax, double tol, int check, double* d_x) {
+  hipStream_t st = c.stream;
+  const int64_t D = S.dim;
+  const size_t vbytes = sizeof(T) * (size_t)D;
+  const bool checked = check > 0 && tol > 0.0;
+  const char* e = std::getenv("EDL_LANCZOS_BASIS");
+  DevBuf basis;
+  if (d_x && !(e && e[0] == '0')) basis = DevBuf::try_alloc(vbytes * (size_t)nmax);
+  // chain descriptor, outputs, norms of the stored vectors and weights, and
+  // (checked) the vectors kept between launches
+  Arena ar;
+  ar.reserve(Arena::round(sizeof(ResChain)) + Arena::round(res_out_bytes(nmax)) +
+             2 * Arena::round(sizeof(double) * nmax) + (checked ? 2 * Arena::round(vbytes) : 0));
+  ResChain r = res_chain<T>(S, nmax);
+  ResChain* d_r = static_cast<ResChain*>(ar.take(sizeof(ResChain)));
+  char* d_out = static_cast<char*>(ar.take(res_out_bytes(nmax)));
+  r.bscale = static_cast<double*>(ar.take(sizeof(double) * nmax));
+  double* d_w = static_cast<double*>(ar.take(sizeof(double) * nmax));
+  r.sc = reinterpret_cast<LzScalars*>(d_out);
+  r.alpha = reinterpret_cast<double*>(d_out + sizeof(LzScalars));
+  r.beta = r.alpha + nmax;
+  r.basis = basis.p;
+  if (checked) {
+    r.q0 = ar.take(vbytes);
+    r.q1 = ar.take(vbytes);
+  }
+  std::vector<char> out(res_out_bytes(nmax));
+  auto launch = [&](const ResChain& rc, int steps) {
+    EDL_HIP(hipMemcpyAsync(d_r, &rc, sizeof(rc), hipMemcpyHostToDevice, st));
+    launch_resident<T>(d_r, 1, D, res_lds_bytes(S, sizeof(T)), res_one(S), c.model.inter, steps, st);
+    EDL_HIP(hipMemcpyAsync(out.data(), d_out, out.size(), hipMemcpyDeviceToHost, st));
+    EDL_HIP(hipStreamSynchronize(st));  // rc and out belong to the host
+  };
+  GsRun g;
+  r.src = d_start;
+  double e_prev = 0.0;
+  bool have_prev = false;
+  for (int done = 0; done < nmax;) {
+    const int n = checked ? std::min(check, nmax - done) : nmax;
+    launch(r, n);
+    done += n;
+    r.src = nullptr;
+    g.hxv += n;
+    if (!checked || n < check) continue;
+    LzScalars sc;
+    std::memcpy(&sc, out.data(), sizeof(sc));
+    if (sc.stopped) break;
+    ChainOut o = res_out(out.data(), nmax);
+    const double e0 = lowest_ritz(o, nullptr);
+    if (have_prev && std::fabs(e0 - e_prev) <= tol * std::fabs(e0)) break;
+    e_prev = e0;
+    have_prev = true;
+  }
+  g.out = res_out(out.data(), nmax);
+  std::vector<double> cvec;
+  g.e0 = lowest_ritz(g.out, d_x ? &cvec : nullptr);
+  if (!d_x) return g;
+  const int m = g.out.nsteps;
+  std::vector<double> w(m);
+  if (basis.p) {
+    EDL_HIP(hipMemcpyAsync(w.data(), r.bscale, sizeof(double) * m, hipMemcpyDeviceToHost, st));
+    EDL_HIP(hipStreamSynchronize(st));
+    for (int k = 0; k < m; ++k) w[k] = cvec[k] / w[k];
+    EDL_HIP(hipMemcpyAsync(d_w, w.data(), sizeof(double) * m, hipMemcpyHostToDevice, st));
+    launch_basis_combine<T>(basis.as<T>(), r.V, d_w, m, d_x, st);
+  } else {
+    EDL_HIP(hipMemcpyAsync(d_w, cvec.data(), sizeof(double) * m, hipMemcpyHostToDevice, st));
+    launch_zero_bytes(d_x, sizeof(double) * D, st);
+    ResChain x = r;
+    x.src = d_start;
+    x.q0 = x.q1 = nullptr;
+    x.x = d_x;
+    x.ccoef = d_w;
+    x.nmax = m;
+    launch(x, m);
+    g.hxv += m;
+  }
+  const double n2 = device_dot(c, d_x, d_x, D, st);
+  launch_scale(d_x, D, 1.0 / std::sqrt(n2), st);
+  EDL_HIP(hipStreamSynchronize(st));
+  return g;
+}
+
 // One ground-state Lanczos run from d_start; the normalised Ritz vector of
 // the lowest eigenvalue is rebuilt into d_x (fp64) by replaying the same
 // deterministic recurrence with the tridiagonal eigenvector as weights.
@@ -1214,6 +1338,8 @@ static GsRun gs_run(Ctx& c, Sector& S, const double* d_start, int niter, double 
                     const double* d_X = nullptr, int nX = 0) {
   hipStream_t st = c.stream;
   const int nmax = (int)std::min<int64_t>(niter, S.dim);
+  if (nX == 0 && resident_sector(S, sizeof(T)))
+    return gs_run_resident<T>(c, S, d_start, nmax, tol, check, d_x);
   GsRun r;
   Schedule sch;
   // Sectors whose columns fit in LDS: the two-pass step (LzChain); larger
@@ -2164,11 +2290,88 @@ static bool bt_pick_persist(Ctx& c, const std::vector<BtChain>& chains, const Bt
   return it->second.first;
 }
 
+// A group of chains whose target sectors all run resident: every seed built,
+// normalised and run by its own block, one launch and one copy back.
+template <typename T>
+static int64_t tridiag_resident(Ctx& c, const std::vector<SeedSpec>& seeds, const std::vector<int>& idx,
+                                const std::vector<int>& targets, int nlanc, double* alpha, double* beta,
+                                double* norm2, int* nsteps, const double* host_seed) {
+  hipStream_t st = c.stream;
+  const size_t n = idx.size();
+  if (n == 0) return 0;
+  std::vector<ResChain> r(n);
+  std::vector<size_t> at(n + 1, 0);
+  int64_t max_dim = 1;
+  size_t lds = 0, src_bytes = 0;
+  bool one = true;
+  for (size_t k = 0; k < n; ++k) {
+    const Sector& J = get_sector(c, targets[idx[k]]);
+    r[k] = res_chain<T>(J, (int)std::min<int64_t>(nlanc, J.dim));
+    at[k + 1] = at[k] + Arena::round(res_out_bytes(r[k].nmax));
+    max_dim = std::max<int64_t>(max_dim, J.dim);
+    lds = std::max(lds, res_lds_bytes(J, sizeof(T)));
+    one = one && res_one(J);
+    if (host_seed || seeds[idx[k]].op == EDL_OP_J) src_bytes += Arena::round(sizeof(double) * (size_t)J.dim);
+  }
+  Arena ar;
+  ar.reserve(Arena::round(at[n]) + Arena::round(sizeof(ResChain) * n) + src_bytes);
+  char* d_out = static_cast<char*>(ar.take(at[n]));
+  ResChain* d_r = static_cast<ResChain*>(ar.take(sizeof(ResChain) * n));
+  int steps = 0;
+  for (size_t k = 0; k < n; ++k) {
+    const SeedSpec& sd = seeds[idx[k]];
+    const Sector& J = get_sector(c, targets[idx[k]]);
+    steps = std::max(steps, r[k].nmax);
+    r[k].sc = reinterpret_cast<LzScalars*>(d_out + at[k]);
+    r[k].alpha = reinterpret_cast<double*>(d_out + at[k] + sizeof(LzScalars));
+    r[k].beta = r[k].alpha + r[k].nmax;
+    if (host_seed || sd.op == EDL_OP_J) {
+      double* src = static_cast<double*>(ar.take(sizeof(double) * (size_t)J.dim));
+      if (host_seed) {
+        EDL_HIP(hipMemcpyAsync(src, host_seed, sizeof(double) * J.dim, hipMemcpyHostToDevice, st));
+      } else {
+        gs_sector_of(c, "edl_tridiag_batched");
+        launch_current_seed(current_terms(c.model, sd.io), c.d_gs, J, src, st);
+      }
+      r[k].src = src;
+    } else {
+      r[k].gs_dimup = gs_sector_of(c, "edl_tridiag_batched").sp[0].dim;
+      r[k].gs = c.d_gs;
+      r[k].seed = sd;
+    }
+  }
+  EDL_HIP(hipMemcpyAsync(d_r, r.data(), sizeof(ResChain) * n, hipMemcpyHostToDevice, st));
+  launch_resident<T>(d_r, (int)n, max_dim, lds, one, c.model.inter, steps, st);
+  std::vector<char> out(at[n]);
+  EDL_HIP(hipMemcpyAsync(out.data(), d_out, at[n], hipMemcpyDeviceToHost, st));
+  EDL_HIP(hipStreamSynchronize(st));
+  int64_t hxv = 0;
+  for (size_t k = 0; k < n; ++k) {
+    const ChainOut o = res_out(out.data() + at[k], r[k].nmax);
+    const size_t s = (size_t)idx[k];
+    for (int j = 0; j < nlanc; ++j) {
+      alpha[s * nlanc + j] = j < r[k].nmax ? o.alpha[j] : 0.0;
+      beta[s * nlanc + j] = j < r[k].nmax ? o.beta[j] : 0.0;
+    }
+    norm2[s] = o.norm2;
+    if (nsteps) nsteps[s] = o.nsteps;
+    hxv += o.nsteps;
+  }
+  return hxv;
+}
+
 template <typename T>
 static int64_t tridiag_group(Ctx& c, const std::vector<SeedSpec>& seeds, const std::vector<int>& idx,
                              const std::vector<int>& targets, int nlanc, double* alpha, double* beta, double* norm2,
                              int* nsteps, const double* host_seed) {
   hipStream_t st = c.stream;
+  {
+    // small targets: resident chains, unless EDL_BATCHED_KERNELS forces a form
+    const char* e = std::getenv("EDL_BATCHED_KERNELS");
+    bool res = !(e && *e);
+    for (size_t k = 0; k < idx.size() && res; ++k) res = resident_sector(get_sector(c, targets[idx[k]]), sizeof(T));
+    if (res) return tridiag_resident<T>(c, seeds, idx, targets, nlanc, alpha, beta, norm2, nsteps, host_seed);
+  }
   std::vector<ChainAlloc<T>> allocs(idx.size());
   std::vector<ChainDev> chains;
   std::vector<BtChain> btchains;

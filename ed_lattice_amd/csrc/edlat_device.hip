@@ -5,4 +5,5 @@
 #include "seeds.hip"
 #include "hxv2.hip"
 #include "batched2.hip"
+#include "resident.hip"
 #include "noalloc.hip"
