@@ -56,38 +56,118 @@ static void release_sectors(Ctx& c) {
   c.sectors.clear();
 }
 
+// ------------------------------------------------------- device memory
+void* DevPool::take(size_t bytes) {
+  // sizes in steps of an eighth, so that buffers of nearly equal calls match
+  size_t step = 512;
+  while (step * 16 <= bytes) step *= 2;
+  const size_t want = (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+  auto it = free_.lower_bound(want);
+  if (it != free_.end() && it->first <= want + want / 4) {
+    void* p = it->second;
+    cached_ -= it->first;
+    live_[p] = it->first;
+    free_.erase(it);
+    return p;
+  }
+  void* p = nullptr;
+  if (hipMalloc(&p, want) != hipSuccess) {
+    (void)hipGetLastError();
+    release();
+    if (hipMalloc(&p, want) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+  }
+  live_[p] = want;
+  return p;
+}
+void DevPool::give(void* p) {
+  if (!p) return;
+  auto it = live_.find(p);
+  if (it == live_.end()) {
+    (void)hipFree(p);
+    return;
+  }
+  const size_t n = it->second;
+  live_.erase(it);
+  if (!bound_) {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) (void)hipGetLastError();
+    bound_ = std::max<size_t>(total_b / 16, 1);
+  }
+  if (cached_ + n > bound_) {
+    (void)hipFree(p);
+    return;
+  }
+  free_.emplace(n, p);
+  cached_ += n;
+}
+void DevPool::release() {
+  for (auto& kv : free_) (void)hipFree(kv.second);
+  free_.clear();
+  cached_ = 0;
+}
+DevPool*& current_pool() {
+  static thread_local DevPool* p = nullptr;
+  return p;
+}
+void* dev_try_alloc(size_t bytes) {
+  if (DevPool* pool = current_pool()) return pool->take(bytes);
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes ? bytes : 4) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return p;
+}
+void* dev_alloc(size_t bytes) {
+  void* p = dev_try_alloc(bytes);
+  if (!p) throw Error("out of device memory (" + std::to_string(bytes) + " bytes)");
+  return p;
+}
+void dev_free(void* p) {
+  if (!p) return;
+  if (DevPool* pool = current_pool())
+    pool->give(p);
+  else
+    (void)hipFree(p);
+}
+
 // ------------------------------------------------------------ utilities
 struct DevBuf {
   void* p = nullptr;
   DevBuf() = default;
-  explicit DevBuf(size_t bytes) { EDL_HIP(hipMalloc(&p, bytes ? bytes : 4)); }
+  explicit DevBuf(size_t bytes) : p(dev_alloc(bytes)) {}
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   DevBuf(DevBuf&& o) noexcept : p(o.p) { o.p = nullptr; }
   DevBuf& operator=(DevBuf&& o) noexcept {
     if (this != &o) {
-      if (p) (void)hipFree(p);
+      dev_free(p);
       p = o.p;
       o.p = nullptr;
     }
     return *this;
   }
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
-  }
+  ~DevBuf() { dev_free(p); }
   template <typename T>
   T* as() const { return static_cast<T*>(p); }
   // An optional allocation: empty (and no error left pending) when the
   // device cannot provide it.
   static DevBuf try_alloc(size_t bytes) {
     DevBuf b;
-    if (hipMalloc(&b.p, bytes ? bytes : 4) != hipSuccess) {
-      b.p = nullptr;
-      (void)hipGetLastError();
-    }
+    b.p = dev_try_alloc(bytes);
     return b;
   }
 };
+
+// Device memory a call can still take: free, or cached by its own context.
+static size_t available_bytes() {
+  size_t free_b = 0, total_b = 0;
+  EDL_HIP(hipMemGetInfo(&free_b, &total_b));
+  return free_b + (current_pool() ? current_pool()->cached() : 0);
+}
 
 // Bump allocator over one device allocation: the buffers of a chain group
 // cost one hipMalloc.
@@ -1394,9 +1474,7 @@ static GsRun gs_run(Ctx& c, Sector& S, const double* d_start, int niter, double 
   bool use_basis = false;
   if (d_x && two && !seg && nX == 0) {
     const char* e = std::getenv("EDL_LANCZOS_BASIS");
-    size_t free_b = 0, total_b = 0;
-    EDL_HIP(hipMemGetInfo(&free_b, &total_b));
-    use_basis = !(e && e[0] == '0') && (double)vbytes * nmax <= 0.7 * (double)free_b;
+    use_basis = !(e && e[0] == '0') && (double)vbytes * nmax <= 0.7 * (double)available_bytes();
   }
   DevBuf basis, bscale;
   if (use_basis) {
@@ -1482,7 +1560,7 @@ static std::map<const Ctx*, GsStats>& gs_stats() {
 
 // Drop the installed state (a new model invalidates it).
 static void clear_gs(Ctx& c) {
-  if (c.d_gs) (void)hipFree(c.d_gs);
+  c.pool.give(c.d_gs);
   c.d_gs = nullptr;
   c.gs_dim = 0;
   c.gs_sector = 0;
@@ -1559,7 +1637,8 @@ extern "C" int edl_ctx_destroy(edl_ctx* ctx) {
   EDL_HIP(hipSetDevice(ctx->c.device));
   EDL_HIP(hipStreamSynchronize(ctx->c.stream));
   release_sectors(ctx->c);
-  if (ctx->c.d_gs) (void)hipFree(ctx->c.d_gs);
+  clear_gs(ctx->c);
+  ctx->c.pool.release();
   if (ctx->c.d_scratch) (void)hipFree(ctx->c.d_scratch);
   for (void* p : ctx->c.user_bufs) (void)hipFree(p);
   (void)hipStreamDestroy(ctx->c.stream);
@@ -1601,6 +1680,7 @@ extern "C" int edl_set_hamiltonian(edl_ctx* ctx, int Ns, int Nspin, int Norb, co
   // the installed state belongs to the previous model
   clear_gs(ctx->c);
   Model& M = ctx->c.model;
+  if (M.Ns != Ns) ctx->c.pool.release();
   M.Ns = Ns;
   M.Nspin = Nspin;
   M.Norb = Norb;
@@ -1705,6 +1785,7 @@ extern "C" int edl_sector_rank(edl_ctx* ctx, int isector, int ispin, int64_t n, 
   API_BEGIN
   EDL_CHECK(ispin == 1 || ispin == 2, "edl_sector_rank: ispin must be 1 or 2");
   EDL_HIP(hipSetDevice(ctx->c.device));
+  PoolScope pool(ctx->c.pool);
   Sector& s = get_sector(ctx->c, isector);
   if (n <= 0) return 0;
   DevBuf ds(sizeof(int32_t) * n), dp(sizeof(int32_t) * n);
@@ -1728,6 +1809,7 @@ extern "C" int edl_hxv(edl_ctx* ctx, int isector, int prec, const void* v, void*
   EDL_CHECK(v && hv, "edl_hxv: null vector");
   EDL_CHECK(prec == EDL_FP64 || prec == EDL_FP32, "edl_hxv: prec must be EDL_FP64 or EDL_FP32");
   EDL_HIP(hipSetDevice(ctx->c.device));
+  PoolScope pool(ctx->c.pool);
   Sector& s = get_sector(ctx->c, isector);
   EventTimer tm(ctx->c.stream);
   if (prec == EDL_FP64)
@@ -1819,6 +1901,7 @@ extern "C" int edl_hxv_host(edl_ctx* ctx, int isector, int prec, const double* v
   EDL_CHECK(v && hv, "edl_hxv_host: null vector");
   EDL_CHECK(prec == EDL_FP64 || prec == EDL_FP32, "edl_hxv_host: prec must be EDL_FP64 or EDL_FP32");
   EDL_HIP(hipSetDevice(ctx->c.device));
+  PoolScope pool(ctx->c.pool);
   Sector& s = get_sector(ctx->c, isector);
   if (prec == EDL_FP64) hxv_host_impl<double>(ctx->c, s, v, hv, 1);
   else hxv_host_impl<float>(ctx->c, s, v, hv, 1);
@@ -1830,6 +1913,7 @@ extern "C" int edl_hxv_host_complex(edl_ctx* ctx, int isector, int prec, const d
   EDL_CHECK(v && hv, "edl_hxv_host_complex: null vector");
   EDL_CHECK(prec == EDL_FP64 || prec == EDL_FP32, "edl_hxv_host_complex: prec must be EDL_FP64 or EDL_FP32");
   EDL_HIP(hipSetDevice(ctx->c.device));
+  PoolScope pool(ctx->c.pool);
   Sector& s = get_sector(ctx->c, isector);
   for (int part = 0; part < 2; ++part) {
     if (prec == EDL_FP64) hxv_host_impl<double>(ctx->c, s, v + part, hv + part, 2);
@@ -1844,6 +1928,7 @@ extern "C" int edl_vec_random(edl_ctx* ctx, int prec, void* dev, int64_t n, uint
   EDL_CHECK(prec == EDL_FP64 || prec == EDL_FP32, "edl_vec_random: prec must be EDL_FP64 or EDL_FP32");
   Ctx& c = ctx->c;
   EDL_HIP(hipSetDevice(c.device));
+  PoolScope pool(ctx->c.pool);
   if (prec == EDL_FP64) {
     launch_start_vector(static_cast<double*>(dev), n, seed, c.stream);
   } else {
@@ -1866,6 +1951,7 @@ extern "C" int edl_vec_dot(edl_ctx* ctx, int prec, const void* a, const void* b,
   EDL_CHECK(prec == EDL_FP64 || prec == EDL_FP32, "edl_vec_dot: prec must be EDL_FP64 or EDL_FP32");
   Ctx& c = ctx->c;
   EDL_HIP(hipSetDevice(c.device));
+  PoolScope pool(ctx->c.pool);
   *out = (prec == EDL_FP64) ? device_dot_t<double>(static_cast<const double*>(a), static_cast<const double*>(b), n, c.stream)
                             : device_dot_t<float>(static_cast<const float*>(a), static_cast<const float*>(b), n, c.stream);
   API_END
@@ -1904,6 +1990,7 @@ extern "C" int edl_lanczos_gs(edl_ctx* ctx, int isector, int prec, int niter, do
   EDL_CHECK(niter >= 1, "edl_lanczos_gs: niter must be >= 1");
   Ctx& c = ctx->c;
   EDL_HIP(hipSetDevice(c.device));
+  PoolScope pool(ctx->c.pool);
   Sector& S = get_sector(c, isector);
   const int64_t D = S.dim;
   hipStream_t st = c.stream;
@@ -1992,6 +2079,7 @@ extern "C" int edl_lanczos_states(edl_ctx* ctx, int isector, int prec, int nstat
   EDL_CHECK(niter >= 1 && nstates >= 1 && energies, "edl_lanczos_states: bad arguments");
   Ctx& c = ctx->c;
   EDL_HIP(hipSetDevice(c.device));
+  PoolScope pool(ctx->c.pool);
   Sector& S = get_sector(c, isector);
   const int64_t D = S.dim;
   EDL_CHECK(nstates <= D, "edl_lanczos_states: more states than the sector dimension");
@@ -2026,6 +2114,7 @@ extern "C" int edl_set_state(edl_ctx* ctx, int isector, double energy, const dou
   EDL_CHECK(vec, "edl_set_state: null vector");
   Ctx& c = ctx->c;
   EDL_HIP(hipSetDevice(c.device));
+  PoolScope pool(ctx->c.pool);
   Sector& S = get_sector(c, isector);
   DevBuf x(sizeof(double) * S.dim);
   EDL_HIP(hipMemcpyAsync(x.p, vec, sizeof(double) * S.dim, hipMemcpyHostToDevice, c.stream));
@@ -2598,6 +2687,7 @@ extern "C" int edl_tridiag(edl_ctx* ctx, int isector, int prec, const double* se
   EDL_CHECK(nlanc >= 1, "edl_tridiag: nlanc must be >= 1");
   Ctx& c = ctx->c;
   EDL_HIP(hipSetDevice(c.device));
+  PoolScope pool(ctx->c.pool);
   get_sector(c, isector);
   std::vector<SeedSpec> seeds(1, SeedSpec{0, 0, 0, 0});
   std::vector<int> idx(1, 0), tg(1, isector);
@@ -2622,6 +2712,7 @@ extern "C" int edl_tridiag_batched(edl_ctx* ctx, int nseeds, const edl_seed_desc
   EDL_CHECK(nlanc >= 1, "edl_tridiag_batched: nlanc must be >= 1");
   Ctx& c = ctx->c;
   EDL_HIP(hipSetDevice(c.device));
+  PoolScope pool(ctx->c.pool);
   gs_sector_of(c, "edl_tridiag_batched");
   const int Ns = c.model.Ns;
   std::vector<SeedSpec> sp(nseeds);
@@ -2649,8 +2740,7 @@ extern "C" int edl_tridiag_batched(edl_ctx* ctx, int nseeds, const edl_seed_desc
   // (each chain holds two stored vectors; one fp64 seed buffer is shared).
   int g = (group <= 0) ? (int)active.size() : group;
   if (group <= 0 && !active.empty()) {
-    size_t free_b = 0, total_b = 0;
-    EDL_HIP(hipMemGetInfo(&free_b, &total_b));
+    const size_t free_b = available_bytes();
     int64_t maxdim = 0;
     for (int s : active) maxdim = std::max<int64_t>(maxdim, get_sector(c, targets[s]).dim);
     // q0, q1 and the two-pass intermediate, with the padded column stride
@@ -2696,6 +2786,7 @@ extern "C" int edl_observables(edl_ctx* ctx, double* dens_up, double* dens_dw, d
   Ctx& c = ctx->c;
   EDL_CHECK(dens_up && dens_dw && docc, "edl_observables: null output");
   EDL_HIP(hipSetDevice(c.device));
+  PoolScope pool(ctx->c.pool);
   Sector& S = gs_sector_of(c, "edl_observables");
   device_observables(c, S, c.d_gs, dens_up, dens_dw, docc);
   API_END
@@ -2706,6 +2797,7 @@ extern "C" int edl_correlations(edl_ctx* ctx, double* sz2, double* n2) {
   Ctx& c = ctx->c;
   EDL_CHECK(sz2 && n2, "edl_correlations: null output");
   EDL_HIP(hipSetDevice(c.device));
+  PoolScope pool(ctx->c.pool);
   Sector& S = gs_sector_of(c, "edl_correlations");
   device_correlations(c, S, c.d_gs, sz2, n2);
   API_END
@@ -2716,6 +2808,7 @@ extern "C" int edl_local_energy(edl_ctx* ctx, double* e) {
   Ctx& c = ctx->c;
   EDL_CHECK(e, "edl_local_energy: null output");
   EDL_HIP(hipSetDevice(c.device));
+  PoolScope pool(ctx->c.pool);
   Sector& S = gs_sector_of(c, "edl_local_energy");
   device_energy(c, S, c.d_gs, e);
   API_END

@@ -446,11 +446,11 @@ BtShape bt_shape(int max_dimup, int max_dimdw, size_t elem) {
 }
 
 BtSet::~BtSet() {
-  if (d) (void)hipFree(d);
-  if (d_tile_up) (void)hipFree(d_tile_up);
-  if (d_tile_dw) (void)hipFree(d_tile_dw);
-  if (d_chain_up) (void)hipFree(d_chain_up);
-  if (d_chain_dw) (void)hipFree(d_chain_dw);
+  dev_free(d);
+  dev_free(d_tile_up);
+  dev_free(d_tile_dw);
+  dev_free(d_chain_up);
+  dev_free(d_chain_dw);
 }
 
 // LDS limits of every instantiation, set once per device and outside any
@@ -493,9 +493,9 @@ void bt_finalize(BtSet& bs) {
   }
   bs.tiles_up = tu[n];
   bs.tiles_dw = td[n];
-  EDL_HIP(hipMalloc(&bs.d, sizeof(BtChain) * n));
-  EDL_HIP(hipMalloc(&bs.d_tile_up, sizeof(int64_t) * (n + 1)));
-  EDL_HIP(hipMalloc(&bs.d_tile_dw, sizeof(int64_t) * (n + 1)));
+  bs.d = static_cast<BtChain*>(dev_alloc(sizeof(BtChain) * n));
+  bs.d_tile_up = static_cast<int64_t*>(dev_alloc(sizeof(int64_t) * (n + 1)));
+  bs.d_tile_dw = static_cast<int64_t*>(dev_alloc(sizeof(int64_t) * (n + 1)));
   EDL_HIP(hipMemcpy(bs.d, bs.h.data(), sizeof(BtChain) * n, hipMemcpyHostToDevice));
   EDL_HIP(hipMemcpy(bs.d_tile_up, tu.data(), sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice));
   EDL_HIP(hipMemcpy(bs.d_tile_dw, td.data(), sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice));
@@ -504,8 +504,8 @@ void bt_finalize(BtSet& bs) {
     for (int64_t t = tu[k]; t < tu[k + 1]; ++t) cu[(size_t)t] = (int32_t)k;
     for (int64_t t = td[k]; t < td[k + 1]; ++t) cdw[(size_t)t] = (int32_t)k;
   }
-  EDL_HIP(hipMalloc(&bs.d_chain_up, sizeof(int32_t) * std::max<size_t>(cu.size(), 1)));
-  EDL_HIP(hipMalloc(&bs.d_chain_dw, sizeof(int32_t) * std::max<size_t>(cdw.size(), 1)));
+  bs.d_chain_up = static_cast<int32_t*>(dev_alloc(sizeof(int32_t) * std::max<size_t>(cu.size(), 1)));
+  bs.d_chain_dw = static_cast<int32_t*>(dev_alloc(sizeof(int32_t) * std::max<size_t>(cdw.size(), 1)));
   EDL_HIP(hipMemcpy(bs.d_chain_up, cu.data(), sizeof(int32_t) * cu.size(), hipMemcpyHostToDevice));
   EDL_HIP(hipMemcpy(bs.d_chain_dw, cdw.data(), sizeof(int32_t) * cdw.size(), hipMemcpyHostToDevice));
 }

@@ -491,35 +491,32 @@ static double host_sum_partials(const double* part, int g, hipStream_t st) {
 
 double device_dot(Ctx& c, const double* a, const double* b, int64_t n, hipStream_t st) {
   const int g = grid_for(n);
-  double* part = nullptr;
-  EDL_HIP(hipMalloc(&part, sizeof(double) * g));
+  double* part = static_cast<double*>(dev_alloc(sizeof(double) * g));
   hipLaunchKernelGGL(k_dot_partial, dim3(g), dim3(kBlock), 0, st, a, b, n, part);
   EDL_HIP(hipGetLastError());
   const double s = host_sum_partials(part, g, st);
-  EDL_HIP(hipFree(part));
+  dev_free(part);
   return s;
 }
 
 template <typename T>
 double device_sumsq(const T* a, int64_t n, hipStream_t st) {
   const int g = grid_for(n);
-  double* part = nullptr;
-  EDL_HIP(hipMalloc(&part, sizeof(double) * g));
+  double* part = static_cast<double*>(dev_alloc(sizeof(double) * g));
   hipLaunchKernelGGL(k_sumsq_partial<T>, dim3(g), dim3(kBlock), 0, st, a, n, part);
   EDL_HIP(hipGetLastError());
   const double s = host_sum_partials(part, g, st);
-  EDL_HIP(hipFree(part));
+  dev_free(part);
   return s;
 }
 template <typename T>
 double device_dot_t(const T* a, const T* b, int64_t n, hipStream_t st) {
   const int g = grid_for(n);
-  double* part = nullptr;
-  EDL_HIP(hipMalloc(&part, sizeof(double) * g));
+  double* part = static_cast<double*>(dev_alloc(sizeof(double) * g));
   hipLaunchKernelGGL(k_dot_partial_t<T>, dim3(g), dim3(kBlock), 0, st, a, b, n, part);
   EDL_HIP(hipGetLastError());
   const double s = host_sum_partials(part, g, st);
-  EDL_HIP(hipFree(part));
+  dev_free(part);
   return s;
 }
 template double device_dot_t<double>(const double*, const double*, int64_t, hipStream_t);
@@ -556,7 +553,7 @@ static int pick_grid(Ctx& c, int64_t total_tiles, const Schedule& w) {
 
 template <typename T>
 ChainSet<T>::~ChainSet() {
-  for (void* p : owned) (void)hipFree(p);
+  for (void* p : owned) dev_free(p);
 }
 
 template <typename T>
@@ -575,17 +572,16 @@ void chainset_finalize(Ctx& c, ChainSet<T>& cs, const Schedule& want) {
   t0[cs.h.size()] = tot;
   cs.sch.total_tiles = tot;
   cs.sch.grid = pick_grid(c, tot, want);
-  double* d_part = nullptr;
-  EDL_HIP(hipMalloc(&d_part, sizeof(double) * (part_total ? part_total : 1)));
+  double* d_part = static_cast<double*>(dev_alloc(sizeof(double) * (part_total ? part_total : 1)));
   cs.owned.push_back(d_part);
   size_t off = 0;
   for (auto& cd : cs.h) {
     cd.part = d_part + off;
     off += (size_t)cd.ntiles;
   }
-  EDL_HIP(hipMalloc(&cs.d, sizeof(ChainDev) * cs.h.size()));
+  cs.d = static_cast<ChainDev*>(dev_alloc(sizeof(ChainDev) * cs.h.size()));
   cs.owned.push_back(cs.d);
-  EDL_HIP(hipMalloc(&cs.d_tile0, sizeof(int64_t) * t0.size()));
+  cs.d_tile0 = static_cast<int64_t*>(dev_alloc(sizeof(int64_t) * t0.size()));
   cs.owned.push_back(cs.d_tile0);
   EDL_HIP(hipMemcpyAsync(cs.d, cs.h.data(), sizeof(ChainDev) * cs.h.size(), hipMemcpyHostToDevice, c.stream));
   EDL_HIP(hipMemcpyAsync(cs.d_tile0, t0.data(), sizeof(int64_t) * t0.size(), hipMemcpyHostToDevice, c.stream));

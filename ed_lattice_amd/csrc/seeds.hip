@@ -12,6 +12,8 @@
 // sign (-1)^popcount(bits below p) is the c/cdg sign of AUX_FUNX.f90:76-102
 // (bits below p agree between source and target).  Up and down operators
 // commute: no sign from the other spin (SECTOR.f90:233-240).
+#include <algorithm>
+
 #include "chains.hpp"
 #include "seeds.hpp"
 
@@ -141,15 +143,41 @@ __global__ void k_colsum(const double* __restrict__ gs, int dimup, int dimdw, do
     colsum[idw] = s;
   }
 }
-__global__ void k_rowsum(const double* __restrict__ gs, int dimup, int dimdw, double* __restrict__ rowsum) {
+// Row sums of |gs|^2 in two launches: blockIdx.y takes one of gridDim.y column
+// chunks (a thread a row, so a wave reads 64 consecutive rows), and the chunks'
+// sums are added in chunk order.  One block column per 256 rows alone left
+// most of the chip idle behind a serial loop over all columns (4x4: 51 blocks).
+__global__ void k_rowsum(const double* __restrict__ gs, int dimup, int dimdw, double* __restrict__ part) {
   const int iup = blockIdx.x * blockDim.x + threadIdx.x;
   if (iup >= dimup) return;
+  const int a = (int)((int64_t)blockIdx.y * dimdw / gridDim.y), e = (int)((int64_t)(blockIdx.y + 1) * dimdw / gridDim.y);
   double v = 0.0;
-  for (int idw = 0; idw < dimdw; ++idw) {
+#pragma unroll 8
+  for (int idw = a; idw < e; ++idw) {
     const double g = gs[(size_t)idw * dimup + iup];
     v += g * g;
   }
+  part[(size_t)blockIdx.y * dimup + iup] = v;
+}
+__global__ void k_rowsum_fold(const double* __restrict__ part, int dimup, int nchunk, double* __restrict__ rowsum) {
+  const int iup = blockIdx.x * blockDim.x + threadIdx.x;
+  if (iup >= dimup) return;
+  double v = 0.0;
+#pragma unroll 8
+  for (int k = 0; k < nchunk; ++k) v += part[(size_t)k * dimup + iup];
   rowsum[iup] = v;
+}
+// Column chunks of the row sums: four blocks a CU in all, at least 16 columns each.
+static int rowsum_chunks(int dimup, int dimdw) {
+  const int bx = (dimup + kBlock - 1) / kBlock;
+  return std::max(1, std::min((dimdw + 15) / 16, 1024 / bx));
+}
+// part: rowsum_chunks * dimup doubles
+static void launch_rowsum(const double* gs, int dimup, int dimdw, double* part, double* rowsum, hipStream_t st) {
+  const int bx = (dimup + kBlock - 1) / kBlock, nch = rowsum_chunks(dimup, dimdw);
+  hipLaunchKernelGGL(k_rowsum, dim3(bx, nch), dim3(kBlock), 0, st, gs, dimup, dimdw, part);
+  hipLaunchKernelGGL(k_rowsum_fold, dim3(bx), dim3(kBlock), 0, st, part, dimup, nch, rowsum);
+  EDL_HIP(hipGetLastError());
 }
 
 void launch_seed(const SeedSpec& s, const double* gs, int gs_dimup, const Sector& target, double* out,
@@ -167,28 +195,27 @@ void device_observables(Ctx& c, const Sector& s, const double* gs, double* dens_
   const int Ns = c.model.Ns;
   hipStream_t st = c.stream;
   const int dimup = s.sp[0].dim, dimdw = s.sp[1].dim;
-  const int nb = 1024;
-  double* part = nullptr;
-  double* rs = nullptr;
-  double* cs = nullptr;
-  EDL_HIP(hipMalloc(&part, sizeof(double) * nb * 32));
-  EDL_HIP(hipMalloc(&rs, sizeof(double) * dimup));
-  EDL_HIP(hipMalloc(&cs, sizeof(double) * dimdw));
+  // blocks of the double occupancy: four elements a thread at least
+  const int nb = (int)std::min<int64_t>(1024, (s.dim + 4 * kBlock - 1) / (4 * kBlock));
+  // {docc partials, row sums, column sums}, one copy back; the row sums' partials after them
+  const size_t n_out = (size_t)nb * 32 + dimup + dimdw;
+  struct Buf {  // freed on every exit, errors included
+    double* p;
+    explicit Buf(size_t n) : p(static_cast<double*>(dev_alloc(sizeof(double) * n))) {}
+    ~Buf() { dev_free(p); }
+  } buf(n_out + (size_t)rowsum_chunks(dimup, dimdw) * dimup);
+  double *part = buf.p, *rs = part + (size_t)nb * 32, *cs = rs + dimup;
   hipLaunchKernelGGL(k_docc<32>, dim3(nb), dim3(kBlock), 0, st, gs, s.sp[0].map, s.sp[1].map, dimup, s.dim, part);
-  hipLaunchKernelGGL(k_rowsum, dim3((dimup + kBlock - 1) / kBlock), dim3(kBlock), 0, st, gs, dimup, dimdw, rs);
+  launch_rowsum(gs, dimup, dimdw, buf.p + n_out, rs, st);
   hipLaunchKernelGGL(k_colsum, dim3(dimdw), dim3(kBlock), 0, st, gs, dimup, dimdw, cs);
   EDL_HIP(hipGetLastError());
-  std::vector<double> hp((size_t)nb * 32), hr(dimup), hc(dimdw);
+  std::vector<double> h(n_out);
   std::vector<int32_t> mu(dimup), md(dimdw);
-  EDL_HIP(hipMemcpyAsync(hp.data(), part, sizeof(double) * hp.size(), hipMemcpyDeviceToHost, st));
-  EDL_HIP(hipMemcpyAsync(hr.data(), rs, sizeof(double) * dimup, hipMemcpyDeviceToHost, st));
-  EDL_HIP(hipMemcpyAsync(hc.data(), cs, sizeof(double) * dimdw, hipMemcpyDeviceToHost, st));
+  EDL_HIP(hipMemcpyAsync(h.data(), part, sizeof(double) * n_out, hipMemcpyDeviceToHost, st));
   EDL_HIP(hipMemcpyAsync(mu.data(), s.sp[0].map, sizeof(int32_t) * dimup, hipMemcpyDeviceToHost, st));
   EDL_HIP(hipMemcpyAsync(md.data(), s.sp[1].map, sizeof(int32_t) * dimdw, hipMemcpyDeviceToHost, st));
   EDL_HIP(hipStreamSynchronize(st));
-  EDL_HIP(hipFree(part));
-  EDL_HIP(hipFree(rs));
-  EDL_HIP(hipFree(cs));
+  const double *hp = h.data(), *hr = hp + (size_t)nb * 32, *hc = hr + dimup;
   for (int p = 0; p < Ns; ++p) {
     double d = 0.0, u = 0.0, w = 0.0;
     for (int b = 0; b < nb; ++b) d += hp[(size_t)b * 32 + p];
@@ -241,22 +268,25 @@ void device_correlations(Ctx& c, const Sector& s, const double* gs, double* sz2,
   hipStream_t st = c.stream;
   const int dimup = s.sp[0].dim, dimdw = s.sp[1].dim;
   struct Buf {  // freed on every exit, errors included
-    double* p = nullptr;
-    explicit Buf(size_t n) { EDL_HIP(hipMalloc(&p, sizeof(double) * n)); }
-    ~Buf() { if (p) (void)hipFree(p); }
-  } rs(dimup), cs(dimdw), A((size_t)32 * dimdw);
-  hipLaunchKernelGGL(k_rowsum, dim3((dimup + kBlock - 1) / kBlock), dim3(kBlock), 0, st, gs, dimup, dimdw, rs.p);
-  hipLaunchKernelGGL(k_colsum, dim3(dimdw), dim3(kBlock), 0, st, gs, dimup, dimdw, cs.p);
-  hipLaunchKernelGGL(k_colbits<32>, dim3(dimdw), dim3(kBlock), 0, st, gs, s.sp[0].map, dimup, A.p);
+    double* p;
+    explicit Buf(size_t n) : p(static_cast<double*>(dev_alloc(sizeof(double) * n))) {}
+    ~Buf() { dev_free(p); }
+  };
+  // {row sums, column sums, up-bit sums}, one copy back; the row sums' partials after them
+  const size_t n_out = (size_t)dimup + 33 * (size_t)dimdw;
+  Buf buf(n_out + (size_t)rowsum_chunks(dimup, dimdw) * dimup);
+  double *rs = buf.p, *cs = rs + dimup, *A = cs + dimdw;
+  launch_rowsum(gs, dimup, dimdw, buf.p + n_out, rs, st);
+  hipLaunchKernelGGL(k_colsum, dim3(dimdw), dim3(kBlock), 0, st, gs, dimup, dimdw, cs);
+  hipLaunchKernelGGL(k_colbits<32>, dim3(dimdw), dim3(kBlock), 0, st, gs, s.sp[0].map, dimup, A);
   EDL_HIP(hipGetLastError());
-  std::vector<double> hr(dimup), hc(dimdw), ha((size_t)32 * dimdw);
+  std::vector<double> h(n_out);
   std::vector<int32_t> mu(dimup), md(dimdw);
-  EDL_HIP(hipMemcpyAsync(hr.data(), rs.p, sizeof(double) * dimup, hipMemcpyDeviceToHost, st));
-  EDL_HIP(hipMemcpyAsync(hc.data(), cs.p, sizeof(double) * dimdw, hipMemcpyDeviceToHost, st));
-  EDL_HIP(hipMemcpyAsync(ha.data(), A.p, sizeof(double) * ha.size(), hipMemcpyDeviceToHost, st));
+  EDL_HIP(hipMemcpyAsync(h.data(), buf.p, sizeof(double) * n_out, hipMemcpyDeviceToHost, st));
   EDL_HIP(hipMemcpyAsync(mu.data(), s.sp[0].map, sizeof(int32_t) * dimup, hipMemcpyDeviceToHost, st));
   EDL_HIP(hipMemcpyAsync(md.data(), s.sp[1].map, sizeof(int32_t) * dimdw, hipMemcpyDeviceToHost, st));
   EDL_HIP(hipStreamSynchronize(st));
+  const double *hr = h.data(), *hc = hr + dimup, *ha = hc + dimdw;
   std::vector<double> uu((size_t)Ns * Ns, 0.0), dd((size_t)Ns * Ns, 0.0), ud((size_t)Ns * Ns, 0.0);
   for (int a = 0; a < dimup; ++a)
     for (int i = 0; i < Ns; ++i)
@@ -364,8 +394,7 @@ void device_energy(Ctx& c, const Sector& s, const double* gs, double* e11) {
       if (io >= 1 && io <= M.Ns) P.u_site[io - 1] = M.Uloc[k];
     }
   const int nb = (int)std::min<int64_t>(1024, (s.dim + 255) / 256);
-  double* part = nullptr;
-  EDL_HIP(hipMalloc(&part, sizeof(double) * 8 * (size_t)nb));
+  double* part = static_cast<double*>(dev_alloc(sizeof(double) * 8 * (size_t)nb));
   hipLaunchKernelGGL(k_energy, dim3(nb), dim3(256), 0, c.stream, gs, s.sp[0].map, s.sp[1].map, s.sp[0].dim,
                      s.sp[1].dim, s.dim, s.sp[0].nbr, s.sp[0].coef64, s.sp[0].cnt, s.sp[1].nbr, s.sp[1].coef64,
                      s.sp[1].cnt, P, part);
@@ -373,7 +402,7 @@ void device_energy(Ctx& c, const Sector& s, const double* gs, double* e11) {
   std::vector<double> h((size_t)nb * 8);
   EDL_HIP(hipMemcpyAsync(h.data(), part, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c.stream));
   EDL_HIP(hipStreamSynchronize(c.stream));
-  EDL_HIP(hipFree(part));
+  dev_free(part);
   double t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   for (int b = 0; b < nb; ++b)
     for (int k = 0; k < 8; ++k) t[k] += h[(size_t)b * 8 + k];

@@ -18,6 +18,13 @@
 
 namespace edl {
 
+// sqrt(x^2 + y^2); the library's hypot, five times as long, only where the
+// squares could leave the range of a double.
+static inline double plane_norm(double x, double y) {
+  const double m = std::max(std::fabs(x), std::fabs(y));
+  return (m < 1e150 && m > 1e-140) ? std::sqrt(x * x + y * y) : std::hypot(x, y);
+}
+
 // d: diagonal [n]; e: off-diagonal, e[i] couples i and i+1 (e[n-1] ignored).
 // On return w holds ascending eigenvalues; Z (n x n, column-major, column j
 // = eigenvector j) if non-null; z1 (first components) if non-null.
@@ -27,7 +34,9 @@ void tridiag_eig(int n, const double* d_in, const double* e_in, double* w, doubl
   for (int i = 0; i + 1 < n; ++i) e[i] = e_in[i];
   const bool full = Z != nullptr;
   const int rows = full ? n : 1;
-  std::vector<double> V((size_t)rows * n, 0.0);  // row-major rows x n
+  // column-major, n columns of `rows`: a rotation runs over two contiguous
+  // columns (row-major, its strided pairs took 4 to 5 times as long at n = 120)
+  std::vector<double> V((size_t)rows * n, 0.0);
   if (full)
     for (int i = 0; i < n; ++i) V[(size_t)i * n + i] = 1.0;
   else
@@ -45,14 +54,14 @@ void tridiag_eig(int n, const double* d_in, const double* e_in, double* w, doubl
       if (++iter > 200) throw std::runtime_error("tridiag_eig: no convergence");
       // Wilkinson-type shift from the leading 2x2 block
       double g = (d[l + 1] - d[l]) / (2.0 * e[l]);
-      double r = std::hypot(g, 1.0);
+      double r = plane_norm(g, 1.0);
       g = d[m] - d[l] + e[l] / (g + std::copysign(r, g));
       double s = 1.0, c = 1.0, p = 0.0;
       int i = m - 1;
       bool deflated = false;
       for (; i >= l; --i) {
         const double f = s * e[i], b = c * e[i];
-        r = std::hypot(f, g);
+        r = plane_norm(f, g);
         e[i + 1] = r;
         if (r == 0.0) {  // underflow: split the matrix here
           d[i + 1] -= p;
@@ -67,11 +76,12 @@ void tridiag_eig(int n, const double* d_in, const double* e_in, double* w, doubl
         p = s * r;
         d[i + 1] = g + p;
         g = c * r - b;
+        double* __restrict__ v0 = &V[(size_t)i * rows];
+        double* __restrict__ v1 = v0 + rows;
         for (int k = 0; k < rows; ++k) {  // rotate columns i, i+1
-          double* row = &V[(size_t)k * n];
-          const double t = row[i + 1];
-          row[i + 1] = s * row[i] + c * t;
-          row[i] = c * row[i] - s * t;
+          const double t = v1[k];
+          v1[k] = s * v0[k] + c * t;
+          v0[k] = c * v0[k] - s * t;
         }
       }
       if (deflated) continue;
@@ -85,10 +95,10 @@ void tridiag_eig(int n, const double* d_in, const double* e_in, double* w, doubl
   std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return d[a] < d[b]; });
   for (int j = 0; j < n; ++j) w[j] = d[ord[j]];
   if (z1)
-    for (int j = 0; j < n; ++j) z1[j] = V[ord[j]];  // row 0
+    for (int j = 0; j < n; ++j) z1[j] = V[(size_t)ord[j] * rows];  // row 0
   if (full)
     for (int j = 0; j < n; ++j)
-      for (int k = 0; k < n; ++k) Z[(size_t)j * n + k] = V[(size_t)k * n + ord[j]];
+      for (int k = 0; k < n; ++k) Z[(size_t)j * n + k] = V[(size_t)ord[j] * n + k];
 }
 
 }  // namespace edl
