@@ -13,6 +13,7 @@
 #include "../../include/edlat_gpu.h"
 #include "batched2.hpp"
 #include "chains.hpp"
+#include "cols.hpp"
 #include "hxv2.hpp"
 #include "resident.hpp"
 #include "seeds.hpp"
@@ -243,9 +244,13 @@ static bool verbose() {
 // two-hop forms exist (one hopping magnitude).  Part of every schedule key:
 // sectors of one shape on lattices of one and of several hopping values share
 // no schedule.
-static int hop_key(const SpinTable& t) { return 2 * t.kmax + (t.nvals == 1 ? 1 : 0); }
+// The non-local block keeps a sector off the one-launch operator.
+static int hop_key(const Sector& s, int spin) {
+  const SpinTable& t = s.sp[spin];
+  return 4 * t.kmax + (t.nvals == 1 ? 1 : 0) + (s.nonlocal ? 2 : 0);
+}
 
-// Tuned operator schedule per (sector shape, column stride, precision), and
+// Tuned operator schedule per (sector shape, column stride, precision, pin), and
 // the chain shapes (the ch_* fields) per (sector shape, precision).
 static std::map<std::tuple<int, int, int, int, int, int>, TwoPassCfg>& tp_cache() {
   static std::map<std::tuple<int, int, int, int, int, int>, TwoPassCfg> m;
@@ -284,6 +289,34 @@ static std::vector<int> dw_chunk_counts(int dimdw, int slots, bool with32 = true
     for (int k : {1, 2}) {
       const int n = (dimdw + k * slots - 1) / (k * slots);
       if (n <= kMaxFitChunks && std::find(v.begin(), v.end(), n) == v.end()) v.push_back(n);
+    }
+  return v;
+}
+
+// The one-launch operator (cols.hpp) is timed against the two passes on vectors
+// of at most this size: at 6.8 MB (3x4 fp64) the two are level, at 35 MB it takes
+// 1.3 times as long.  EDL_ONE_PASS=0|1 keeps it off, or takes it wherever its
+// panels fit.
+constexpr size_t kOnePassBytes = (size_t)16 << 20;
+static int one_pass_pin() {
+  const char* e = std::getenv("EDL_ONE_PASS");
+  return e && *e ? std::atoi(e) : -1;
+}
+// Element size and pin: a changed pin takes a schedule of its own.
+static int one_pass_key(size_t elem) { return (int)elem + 16 * (one_pass_pin() + 1); }
+static bool one_pass_size(const Sector& s, size_t elem) {
+  const int pin = one_pass_pin();
+  return !s.nonlocal && pin != 0 && (pin == 1 || (size_t)s.dim * elem <= kOnePassBytes);
+}
+static std::vector<TwoPassCfg> one_pass_shapes(const TwoPassView& V, const TwoPassCfg& base, size_t elem) {
+  std::vector<TwoPassCfg> v;
+  for (int C : {1, 2, 4})
+    for (int th : {64, 128, 256, 512, 1024}) {
+      if (!cols_ok(V, C, elem) || (th > 64 && th >= 2 * V.dimup)) continue;
+      TwoPassCfg w = base;
+      w.one_C = C;
+      w.one_threads = th;
+      v.push_back(w);
     }
   return v;
 }
@@ -353,7 +386,7 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s, int ld) {
   if (two_pass_pin<T>(V, best)) return best;
   // (layouts of different strides tune apart: the down pass prefers other
   // shapes where its row segments straddle cache lines)
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s.sp[0]), hop_key(s.sp[1]), ld, (int)sizeof(T));
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s, 0), hop_key(s, 1), ld, one_pass_key(sizeof(T)));
   auto it = tp_cache().find(key);
   if (it != tp_cache().end()) return it->second;
   hipStream_t st = c.stream;
@@ -477,6 +510,27 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s, int ld) {
           }
         }
   }
+  // the one-launch form against the two passes together
+  if (one_pass_size(s, sizeof(T))) {
+    auto two = [&]() {
+      launch_pass_up<T>(V, c.model.inter, lut_dev<T>(s.sp[0]), q.as<T>(), q.as<T>(), t.as<T>(), nullptr, best, st);
+      launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), q.as<T>(), q.as<T>(), t.as<T>(), o.as<T>(), nullptr, best, st);
+    };
+    double best_ms = one_pass_pin() == 1 ? 1e300 : std::min(timed(two, 1e300), timed(two, 1e300));
+    for (const TwoPassCfg& w : one_pass_shapes(V, best, sizeof(T))) {
+      const double ms = timed([&]() {
+        launch_cols<T>(V, c.model.inter, lut_dev<T>(s.sp[0]), lut_dev<T>(s.sp[1]), q.as<T>(), o.as<T>(), w, st);
+      }, best_ms);
+      if (verbose())
+        std::fprintf(stderr, "[edl] tune one launch fp%d C %d threads %4d (best so far %.4f): %.4f ms\n",
+                     8 * (int)sizeof(T), w.one_C, w.one_threads, best_ms, ms);
+      if (ms < best_ms) {
+        best_ms = ms;
+        best.one_C = w.one_C;
+        best.one_threads = w.one_threads;
+      }
+    }
+  }
   tp_cache()[key] = best;
   return best;
 }
@@ -486,7 +540,7 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s, int ld) {
 // the operator's, which a pin may set (with_chain_shapes).
 template <typename T>
 static TwoPassCfg two_pass_chain_cfg(Ctx& c, const Sector& s) {
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s.sp[0]), hop_key(s.sp[1]), (int)sizeof(T));
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s, 0), hop_key(s, 1), (int)sizeof(T));
   const int ld = padded_ld(s.sp[0].dim);
   const TwoPassView V = two_pass_view(s, ld);
   TwoPassCfg best;
@@ -700,7 +754,7 @@ static TwoPassCfg seg_cfg(Ctx& c, Sector& s, int ld) {
   static std::map<std::tuple<int, int, int, int, int, int, int, int, int>, TwoPassCfg> cache;
   const int pin = (seg_rank_pin() == 1 && !seg_rank_ok(s)) ? 0 : seg_rank_pin();
   const int cpin = seg_cols_pin();
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s.sp[0]), hop_key(s.sp[1]), ld, (int)sizeof(T),
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s, 0), hop_key(s, 1), ld, (int)sizeof(T),
                                    seg_row_cap(sizeof(T), 1), 2 * pin + (seg_rank_ok(s) ? 1 : 0), cpin);
   auto it = cache.find(key);
   if (it != cache.end()) return it->second;
@@ -865,6 +919,10 @@ static void apply_h(Ctx& c, Sector& s, const T* v, T* out, int ld, hipStream_t s
     launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), vin, vin, tmp, out, nullptr, cfg, st);
   } else if (two_pass_ok(s, sizeof(T))) {
     const TwoPassCfg cfg = two_pass_cfg<T>(c, s, ld);
+    if (cfg.one_C > 0) {
+      launch_cols<T>(two_pass_view(s, ld), c.model.inter, lut_dev<T>(s.sp[0]), lut_dev<T>(s.sp[1]), v, out, cfg, st);
+      return;
+    }
     T* tmp = static_cast<T*>(scratch(c, sizeof(T) * (size_t)ld * s.sp[1].dim));
     const TwoPassView V = two_pass_view(s, ld);
     T* vin = const_cast<T*>(v);  // operator mode only reads it
@@ -1641,6 +1699,8 @@ extern "C" int edl_ctx_destroy(edl_ctx* ctx) {
   ctx->c.pool.release();
   if (ctx->c.d_scratch) (void)hipFree(ctx->c.d_scratch);
   for (void* p : ctx->c.user_bufs) (void)hipFree(p);
+  for (hipEvent_t e : ctx->c.ev)
+    if (e) (void)hipEventDestroy(e);
   (void)hipStreamDestroy(ctx->c.stream);
   gs_stats().erase(&ctx->c);
   delete ctx;
@@ -1811,13 +1871,22 @@ extern "C" int edl_hxv(edl_ctx* ctx, int isector, int prec, const void* v, void*
   EDL_HIP(hipSetDevice(ctx->c.device));
   PoolScope pool(ctx->c.pool);
   Sector& s = get_sector(ctx->c, isector);
-  EventTimer tm(ctx->c.stream);
+  Ctx& c = ctx->c;
+  for (hipEvent_t& e : c.ev)
+    if (!e) EDL_HIP(hipEventCreate(&e));
+  // (kept events and a wait for the stream: 22.3 us around a 10 us kernel, against
+  // 24.9 with events made for the call and a wait for the second)
+  EDL_HIP(hipEventRecord(c.ev[0], c.stream));
   if (prec == EDL_FP64)
-    apply_h<double>(ctx->c, s, (const double*)v, (double*)hv, s.sp[0].dim, ctx->c.stream);
+    apply_h<double>(c, s, (const double*)v, (double*)hv, s.sp[0].dim, c.stream);
   else
-    apply_h<float>(ctx->c, s, (const float*)v, (float*)hv, s.sp[0].dim, ctx->c.stream);
-  ctx->c.last_ms = tm.stop();
-  ctx->c.last_hxv = 1;
+    apply_h<float>(c, s, (const float*)v, (float*)hv, s.sp[0].dim, c.stream);
+  EDL_HIP(hipEventRecord(c.ev[1], c.stream));
+  EDL_HIP(hipStreamSynchronize(c.stream));
+  float ms = 0.f;
+  EDL_HIP(hipEventElapsedTime(&ms, c.ev[0], c.ev[1]));
+  c.last_ms = ms;
+  c.last_hxv = 1;
   API_END
 }
 
@@ -1834,7 +1903,7 @@ static void hxv_noalloc_impl(Ctx& c, Sector& s, const T* v, T* hv) {
   EDL_CHECK(bytes <= noalloc_scratch_bytes(),
             "edl_hxv_noalloc: the sector's intermediate (" + std::to_string(bytes) +
                 " bytes) exceeds the 256 MiB scratch; use edl_hxv");
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s.sp[0]), hop_key(s.sp[1]), ld, (int)sizeof(T));
+  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s, 0), hop_key(s, 1), ld, one_pass_key(sizeof(T)));
   TwoPassCfg cfg;
   auto it = tp_cache().find(key);
   if (it != tp_cache().end()) {
@@ -1855,6 +1924,11 @@ static void hxv_noalloc_impl(Ctx& c, Sector& s, const T* v, T* hv) {
   const TwoPassView V = two_pass_view(s, ld);
   T* tmp = static_cast<T*>(noalloc_scratch(c.device));
   T* vin = const_cast<T*>(v);  // operator mode only reads it
+  if (cfg.one_C > 0) {
+    launch_cols<T>(V, c.model.inter, lut_dev<T>(s.sp[0]), lut_dev<T>(s.sp[1]), v, hv, cfg, c.stream);
+    EDL_HIP(hipStreamSynchronize(c.stream));
+    return;
+  }
   launch_pass_up<T>(V, c.model.inter, lut_dev<T>(s.sp[0]), vin, vin, tmp, nullptr, cfg, c.stream);
   launch_nonlocal<T>(V, c.model.inter, vin, vin, tmp, nullptr, c.stream);
   launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), vin, vin, tmp, hv, nullptr, cfg, c.stream);
@@ -2856,8 +2930,9 @@ template <typename T>
 static void bench_passes_impl(Ctx& c, Sector& s, int reps, double* ms_pass, int32_t* cfg) {
   hipStream_t st = c.stream;
   const bool seg = seg_path(s, sizeof(T));
-  const bool two = !seg && two_pass_ok(s, sizeof(T));
   const int ld = engine_ld<T>(s);
+  // (a sector that runs the one-launch form is reported as a single pass)
+  const bool two = !seg && two_pass_ok(s, sizeof(T)) && two_pass_cfg<T>(c, s, ld).one_C == 0;
   const int64_t D = s.dim, Dp = (int64_t)ld * s.sp[1].dim;
   DevBuf d64(sizeof(double) * D), v(sizeof(T) * Dp), h(sizeof(T) * Dp);
   launch_start_vector(d64.as<double>(), D, 0x5EEDull, st);

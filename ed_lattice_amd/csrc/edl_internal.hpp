@@ -273,6 +273,8 @@ struct Ctx {
   // timing of the last operator / Lanczos call (HIP events on `stream`)
   double last_ms = 0.0;
   int64_t last_hxv = 0;
+  // events of the operator calls, made on first use
+  hipEvent_t ev[2] = {};
   // buffers handed out by edl_device_alloc
   std::vector<void*> user_bufs;
   // buffers of earlier calls (the installed state's among them while it is installed)

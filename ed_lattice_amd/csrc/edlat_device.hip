@@ -6,4 +6,5 @@
 #include "hxv2.hip"
 #include "batched2.hip"
 #include "resident.hip"
+#include "cols.hip"
 #include "noalloc.hip"

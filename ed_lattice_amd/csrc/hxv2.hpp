@@ -96,6 +96,8 @@ struct TwoPassCfg {
                         //    (R 32|64, threads_dw; ncol, kch, nchunk, dw_vec unused)
   int seg_rank = 0;     // segmented sectors, 1: the up pass finds hop targets by rank arithmetic
                         //    (RankHops) instead of reading the hop table
+  int one_C = 0;        // > 0: one launch over panels of that many columns (cols.hpp) instead of
+  int one_threads = 0;  // the two passes; its block size
   int dw_ord = 0;       // 1: the vector-gather down pass takes its columns in the locality order
                         //    (SpinTable::ord; the layout of the vectors is unchanged)
   // Down-pass shape of the Lanczos chains (the pass with the Lanczos terms
