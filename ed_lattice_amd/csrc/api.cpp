@@ -1109,16 +1109,38 @@ struct TwoPassStep {
   double* defl_coef = nullptr;
 };
 
-// EDL_GRAPHS=0: the steps are launched directly, one launch per kernel and
-// step, instead of replaying a captured graph (same kernels and arguments;
-// for tools that collect per-dispatch counters).
+// The buffers a chain's steps share: the two-pass intermediate, the partial
+// sums and, for two-launch steps, the second place of the scalars (after
+// part_dw).
+template <typename T>
+static void chain_buffers(Ctx& c, TwoPassStep<T>& tps, bool seg, bool deflate, const Sector& S, DevBuf& up,
+                          DevBuf& dw) {
+  tps.tmp = static_cast<T*>(scratch(c, sizeof(T) * (size_t)tps.V.ld * S.sp[1].dim));
+  const bool phase_b = seg || deflate;
+  const int nup = phase_b ? phase_b_grid(tps.V) : pass_up_grid(tps.V, tps.cfg), ndw = pass_dw_grid(tps.V, tps.cfg);
+  up = DevBuf(sizeof(double) * nup);
+  dw = DevBuf(sizeof(double) * ndw + sizeof(LzScalars));
+  tps.L.part_up = up.as<double>();
+  tps.L.part_dw = dw.as<double>();
+  if (!phase_b && !S.nonlocal && chain_fused(tps.V, tps.cfg)) {
+    tps.L.sc2 = reinterpret_cast<LzScalars*>(tps.L.part_dw + ndw);
+    tps.L.nup = nup;
+    tps.L.ndw = ndw;
+  }
+}
+
+// EDL_GRAPHS=1: the steps replay a graph captured once instead of being
+// launched directly (same kernels and arguments).  Direct launches are the
+// faster of the two on the box: the host enqueues a step's few kernels in less
+// than they run, and a graph launch per step left a gap between steps (3x4 ground
+// state, 120 steps: 6.04 ms replayed, 5.57 ms direct; 12 fp32 chains 5.46, 5.26).
 static bool graphs_enabled() {
   const char* e = std::getenv("EDL_GRAPHS");
-  return !(e && std::strcmp(e, "0") == 0);
+  return e && std::strcmp(e, "1") == 0;
 }
 
 // Replays `enqueue` (the launches of one step, all on `st`) through a graph
-// captured once, or launches it directly when graphs are off.
+// captured once, or launches it directly (the default).
 struct StepRunner {
   hipStream_t st;
   hipGraph_t g = nullptr;
@@ -1162,6 +1184,7 @@ struct StepRunner {
 template <typename T>
 static int run_steps(Ctx& c, ChainSet<T>& cs, int steps, int check, double tol, hipStream_t st,
                      const TwoPassStep<T>* tp = nullptr) {
+  const bool fused = tp && tp->L.sc2;
   auto enqueue = [&]() {
     if (tp && (tp->seg || tp->nx > 0)) {
       // phase B of the previous step (+ deflation), beta, up (segmented, or the
@@ -1183,11 +1206,12 @@ static int run_steps(Ctx& c, ChainSet<T>& cs, int steps, int check, double tol, 
       // up (+ phase B of the previous step), beta, down (+ phase A), alpha
       T* q0 = static_cast<T*>(cs.h[0].q0);
       T* q1 = static_cast<T*>(cs.h[0].q1);
+      // (two-launch steps: the passes do the scalars' work)
       launch_pass_up<T>(tp->V, c.model.inter, tp->lut_up, q0, q1, tp->tmp, &tp->L, tp->cfg, st);
-      launch_lz_beta(tp->L, tp->V, tp->cfg, st);
+      if (!fused) launch_lz_beta(tp->L, tp->V, tp->cfg, st);
       launch_nonlocal<T>(tp->V, c.model.inter, q0, q1, tp->tmp, &tp->L, st);
       launch_pass_dw<T>(tp->V, tp->lut_dw, q0, q1, tp->tmp, nullptr, &tp->L, tp->cfg, st);
-      launch_lz_alpha(tp->L, tp->V, tp->cfg, st);
+      if (!fused) launch_lz_alpha(tp->L, tp->V, tp->cfg, st);
     } else {
       lz_phase_a(c, cs, st);
       lz_phase_b(c, cs, st);
@@ -1201,6 +1225,7 @@ static int run_steps(Ctx& c, ChainSet<T>& cs, int steps, int check, double tol, 
     run.launch();
     ++done;
     if (check > 0 && tol > 0.0 && (k + 1) % check == 0 && cs.h.size() == 1) {
+      if (fused) launch_lz_alpha(tp->L, tp->V, tp->cfg, st);
       LzScalars s{};
       EDL_HIP(hipMemcpyAsync(&s, cs.h[0].sc, sizeof(s), hipMemcpyDeviceToHost, st));
       EDL_HIP(hipStreamSynchronize(st));
@@ -1217,6 +1242,8 @@ static int run_steps(Ctx& c, ChainSet<T>& cs, int steps, int check, double tol, 
       have_prev = true;
     }
   }
+  // (after a checked step the same sums again)
+  if (fused && done > 0) launch_lz_alpha(tp->L, tp->V, tp->cfg, st);
   EDL_HIP(hipStreamSynchronize(st));
   return done;
 }
@@ -1237,7 +1264,7 @@ static bool batched_chain_forced() {
 static constexpr int64_t kChainAloneDim = 50000000;
 
 // `steps` Lanczos steps of every chain: up pass (with the previous step's
-// phase B), down pass + phase A; captured once as a graph and replayed.
+// phase B), down pass + phase A.
 template <typename T>
 static int run_steps_bt(Ctx& c, const BtSet& bs, int steps, hipStream_t st) {
   StepRunner run(st, [&]() {
@@ -1283,7 +1310,7 @@ struct AuxStream {
 };
 
 // `steps` steps of independent chain sets, part 0 on `st` and each other
-// part on a stream of its own, each replayed from its own graph, launched
+// part on a stream of its own, the parts' steps launched
 // in turn; `st` waits for all of them.
 template <typename T>
 static int run_steps_btn(Ctx& c, const std::vector<BtSet>& parts, int steps, hipStream_t st) {
@@ -1497,11 +1524,7 @@ static GsRun gs_run(Ctx& c, Sector& S, const double* d_start, int niter, double 
     tps.V = two_pass_view(S, ld);
     tps.lut_up = lut_dev<T>(S.sp[0]);
     tps.lut_dw = lut_dev<T>(S.sp[1]);
-    tps.tmp = static_cast<T*>(scratch(c, sizeof(T) * (size_t)ld * S.sp[1].dim));
-    tp_up = DevBuf(sizeof(double) * std::max(phase_b_grid(tps.V), pass_up_grid(tps.V, tps.cfg)));
-    tp_dw = DevBuf(sizeof(double) * pass_dw_grid(tps.V, tps.cfg));
-    tps.L.part_up = tp_up.as<double>();
-    tps.L.part_dw = tp_dw.as<double>();
+    chain_buffers<T>(c, tps, seg, nX > 0, S, tp_up, tp_dw);
     sch.block_threads = 256;
     sch.grid = c.num_cu * 8;
   }
@@ -2697,11 +2720,8 @@ static int64_t tridiag_group(Ctx& c, const std::vector<SeedSpec>& seeds, const s
       tps.V = two_pass_view(J, chains[k].ld);
       tps.lut_up = lut_dev<T>(J.sp[0]);
       tps.lut_dw = lut_dev<T>(J.sp[1]);
-      tps.tmp = static_cast<T*>(scratch(c, sizeof(T) * (size_t)chains[k].ld * J.sp[1].dim));
-      DevBuf pu(sizeof(double) * (seg ? phase_b_grid(tps.V) : pass_up_grid(tps.V, tps.cfg)));
-      DevBuf pd(sizeof(double) * pass_dw_grid(tps.V, tps.cfg));
-      tps.L.part_up = pu.as<double>();
-      tps.L.part_dw = pd.as<double>();
+      DevBuf pu, pd;
+      chain_buffers<T>(c, tps, seg, false, J, pu, pd);
       tps.L.sc = chains[k].sc;
       tps.L.alpha = chains[k].alpha;
       tps.L.beta = chains[k].beta;

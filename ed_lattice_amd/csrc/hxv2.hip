@@ -90,6 +90,21 @@ static __device__ __forceinline__ double flip_sign(double h, uint32_t sbit) {
   return __longlong_as_double(__double_as_longlong(h) ^ ((long long)sbit << 32));
 }
 
+// Sum of part[0 .. n) in every thread of the block: a contiguous slice a
+// thread, the threads' sums by block_sum.
+static __device__ double block_sum_of(const double* __restrict__ part, int n, double* sh) {
+  const int per = (n + (int)blockDim.x - 1) / (int)blockDim.x;
+  const int a = (int)threadIdx.x * per, e = min(a + per, n);
+  double x = 0.0;
+  for (int k = a; k < e; ++k) x += part[k];
+  x = block_sum(x, sh);
+  if (threadIdx.x == 0) sh[0] = x;
+  __syncthreads();
+  x = sh[0];
+  __syncthreads();  // sh is free again
+  return x;
+}
+
 // ------------------------------------------------------------------ pass U
 // One panel of C columns starting at c0: stage them in LDS (interleaved by
 // row), then T(:, c0+j) = [D + H_up] q(:, c0+j) * ts for every row.  Both
@@ -439,7 +454,21 @@ static __device__ __forceinline__ void pass_up_body(const TwoPassView& V, const 
       up_panel<T, C, RPT, UKCH, LREG, COL, H16, SGN>(V, I, lut, P, qa, tout, pan * C, (T)1);
     return;
   }
-  const LzScalars s = *L.sc;
+  LzScalars s = *L.sc;
+  if (L.sc2) {
+    // two-launch steps: alpha of the step before, the scalars to the down pass
+    if (!s.stopped && s.pad == 3) {
+      s.alpha_k = block_sum_of(L.part_dw, L.ndw, sh);
+      s.nsteps = s.k + 1;
+      s.pad = 1;
+      if (blockIdx.x == 0 && threadIdx.x == 0) L.alpha[s.k] = s.alpha_k;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      LzScalars n = s;
+      if (s.pad && s.k + 1 >= L.nmax) n.stopped = 1;
+      *L.sc2 = n;
+    }
+  }
   if (s.stopped) return;
   const bool pend = s.pad != 0;
   const bool last = pend && s.k + 1 >= L.nmax;
@@ -662,7 +691,31 @@ __global__ __launch_bounds__(1024) void k_pass_dwv(TwoPassView V, const T* __res
   const T* __restrict__ q = qa;
   T* __restrict__ out = outp;
   if (MODE == 1) {
-    s = *A.sc;
+    if (A.sc2) {
+      // two-launch steps: beta of this step, the scalars to the next up pass
+      s = *A.sc2;
+      const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+      if (!s.stopped && s.pad) {
+        const double bt = sqrt(block_sum_of(A.part_up, A.nup, sh));
+        if (lead) A.beta[s.k + 1] = bt;
+        s.pad = 0;
+        if (!(bt > A.brk_tol * (fabs(s.alpha_k) + s.beta_k))) {
+          s.stopped = 1;
+        } else {
+          s.s_old = s.s_cur;
+          s.s_cur = bt;
+          s.beta_k = bt;
+          s.k += 1;
+        }
+      }
+      if (lead) {
+        LzScalars n = s;
+        if (!s.stopped) n.pad = 3;
+        *A.sc = n;
+      }
+    } else {
+      s = *A.sc;
+    }
     if (s.stopped) return;
     q = (s.k & 1) ? qb : qa;
     out = (s.k & 1) ? qa : qb;
@@ -1682,6 +1735,11 @@ int pass_dw_grid(const TwoPassView& V, const TwoPassCfg& cfg) {
   if (cfg.dw_vec == 1 && cfg.dw_rng == 0) return (int)(8 * (((int64_t)npan * cfg.nchunk + 7) / 8));
   if (cfg.dw_rng > 0) return 8 * V.rng_n[cfg.dw_rng] * ((npan + 7) / 8);
   return 8 * cfg.nchunk * ((npan + 7) / 8);
+}
+
+constexpr int kFusedBlocks = 2048;
+bool chain_fused(const TwoPassView& V, const TwoPassCfg& cfg) {
+  return cfg.dw_vec == 1 && cfg.dw_rng == 0 && pass_dw_grid(V, cfg) <= kFusedBlocks;
 }
 
 static size_t pass_dwr_lds(const TwoPassView& V, int R, int b, size_t elem) {

@@ -49,7 +49,8 @@ struct TwoPassView {
   int rng_maxwords[kMaxRangeBits + 1];
 };
 
-// One Lanczos chain driven by the two passes.  A step is four launches:
+// One Lanczos chain driven by the two passes.  A step is four launches, or two
+// (sc2 set, see chain_fused):
 //   up     phase B of the previous step where pending (r = t - alpha v over
 //          t, block partials of |r|^2, replay term x += c v), then
 //          T = [D + H_up] q, unscaled;
@@ -59,6 +60,12 @@ struct TwoPassView {
 //          block partials of alpha_k;
 //   alpha  one block: alpha_k, phase B of step k pending.
 // No fence inside the passes: the kernel boundaries publish the partials.
+// With sc2 set, the passes do the beta and alpha launches' work themselves: every
+// block adds the other pass's partials up (in the same order, so all blocks have
+// the same bits), and block 0 hands the scalars on, from sc (down pass to up
+// pass) to sc2 (up pass to down pass).  LzScalars::pad then says 0 no phase B
+// pending (first step), 1 pending with alpha_k known, 3 pending with alpha_k
+// still in part_dw; launch_lz_alpha after the last step completes alpha_k.
 struct LzChain {
   LzScalars* sc;
   double* alpha;          // [nmax]
@@ -71,6 +78,8 @@ struct LzChain {
   double* bscale;         // [nmax] their norms s_k
   int nmax;
   double brk_tol;         // relative breakdown threshold on beta
+  LzScalars* sc2;         // second place of the scalars, or null: four launches a step
+  int nup, ndw;           // blocks of the up and the down pass (with sc2)
 };
 
 struct TwoPassCfg {
@@ -131,6 +140,13 @@ inline TwoPassCfg chain_cfg(const TwoPassCfg& c) {
   }
   return r;
 }
+
+// Whether a chain with this schedule runs steps of two launches: the
+// vector-gather down pass, and few enough blocks that each can add up the other
+// pass's partials.  Below the limit the two small launches cost more than the
+// sums (3x4, 853 776 states, 464 + 512 blocks); a block of the 4x4 sector's
+// 20 000 and more would spend its time on them.
+bool chain_fused(const TwoPassView& V, const TwoPassCfg& cfg);
 
 // Whether the bank-scheduled up-pass table exists for panels of C columns of
 // T (staged rows of an odd number of dwords: fp32 with C = 1 or 3), in the
