@@ -950,18 +950,39 @@ struct ChainOut {
 template <typename T>
 struct ChainAlloc {
   DevBuf q0, q1, sc, alpha, beta, counter;
-  Arena* ar = nullptr;  // carve from this instead of allocating, when set
-  void* get(DevBuf& slot, size_t bytes) {
-    if (ar) return ar->take(bytes);
+  // carve the vectors, and the scalars and coefficients, from these instead of
+  // allocating, when set
+  Arena* ar = nullptr;
+  Arena* small = nullptr;
+  static void* get(Arena* from, DevBuf& slot, size_t bytes) {
+    if (from) return from->take(bytes);
     slot = DevBuf(bytes);
     return slot.p;
   }
   // arena bytes of one chain of D stored elements and nmax steps
-  static size_t arena_bytes(int64_t D, int nmax) {
-    return 2 * Arena::round(sizeof(T) * D) + Arena::round(sizeof(LzScalars)) +
-           2 * Arena::round(sizeof(double) * nmax) + Arena::round(sizeof(unsigned));
+  static size_t vector_bytes(int64_t D) { return 2 * Arena::round(sizeof(T) * D); }
+  static size_t small_bytes(int nmax) {
+    return Arena::round(sizeof(LzScalars)) + 2 * Arena::round(sizeof(double) * nmax) + Arena::round(sizeof(unsigned));
   }
 };
+
+// The vectors, scalars and coefficients of one chain, placed but not written.
+template <typename T>
+static void place_chain(ChainDev& cd, ChainAlloc<T>& A, const Sector& S, int nmax, int ld) {
+  const int64_t D = (int64_t)ld * S.sp[1].dim;
+  fill_sector_view(S, sizeof(T) == 4, cd);
+  cd.ld = ld;
+  cd.q0 = A.get(A.ar, A.q0, sizeof(T) * D);
+  cd.q1 = A.get(A.ar, A.q1, sizeof(T) * D);
+  cd.x = nullptr;
+  cd.ccoef = nullptr;
+  cd.sc = static_cast<LzScalars*>(A.get(A.small, A.sc, sizeof(LzScalars)));
+  cd.alpha = static_cast<double*>(A.get(A.small, A.alpha, sizeof(double) * nmax));
+  cd.beta = static_cast<double*>(A.get(A.small, A.beta, sizeof(double) * nmax));
+  cd.counter = static_cast<unsigned*>(A.get(A.small, A.counter, sizeof(unsigned)));
+  cd.nmax = nmax;
+  cd.brk_tol = 1e-14;
+}
 
 // d_start is in the natural layout; the stored vectors get column stride ld
 // (the padding rows are zero and no kernel writes them).
@@ -974,20 +995,14 @@ static void init_chain(Ctx& c, ChainDev& cd, ChainAlloc<T>& A, const Sector& S, 
                        int64_t part_n = 0) {
   if (ld == 0) ld = S.sp[0].dim;
   const int64_t D = (int64_t)ld * S.sp[1].dim;
-  fill_sector_view(S, sizeof(T) == 4, cd);
-  cd.ld = ld;
-  T* q0 = static_cast<T*>(A.get(A.q0, sizeof(T) * D));
-  T* q1 = static_cast<T*>(A.get(A.q1, sizeof(T) * D));
-  LzScalars* sc = static_cast<LzScalars*>(A.get(A.sc, sizeof(LzScalars)));
-  double* alpha = static_cast<double*>(A.get(A.alpha, sizeof(double) * nmax));
-  double* beta = static_cast<double*>(A.get(A.beta, sizeof(double) * nmax));
-  unsigned* counter = static_cast<unsigned*>(A.get(A.counter, sizeof(unsigned)));
+  place_chain(cd, A, S, nmax, ld);
+  T* q0 = static_cast<T*>(cd.q0);
   if (ld != S.sp[0].dim) launch_zero_bytes(q0, sizeof(T) * D, st);
   launch_convert_ld<T>(d_start, q0, S.sp[0].dim, S.sp[1].dim, ld, st);
-  launch_zero_bytes(q1, sizeof(T) * D, st);
-  launch_zero_bytes(alpha, sizeof(double) * nmax, st);
-  launch_zero_bytes(beta, sizeof(double) * nmax, st);
-  launch_zero_bytes(counter, 4, st);
+  launch_zero_bytes(cd.q1, sizeof(T) * D, st);
+  launch_zero_bytes(cd.alpha, sizeof(double) * nmax, st);
+  launch_zero_bytes(cd.beta, sizeof(double) * nmax, st);
+  launch_zero_bytes(cd.counter, 4, st);
   if (d_ss) {
     EDL_CHECK(part_n >= partials_size(D), "init_chain: partial-sum buffer smaller than the launch grid");
     device_sumsq_to<T>(q0, D, part, d_ss, st);
@@ -1002,20 +1017,10 @@ static void init_chain(Ctx& c, ChainDev& cd, ChainAlloc<T>& A, const Sector& S, 
     s.beta_k = 0.0;
     s.alpha_k = 0.0;
     s.norm2 = norm2;
-    EDL_HIP(hipMemcpyAsync(sc, &s, sizeof(s), hipMemcpyHostToDevice, st));
+    EDL_HIP(hipMemcpyAsync(cd.sc, &s, sizeof(s), hipMemcpyHostToDevice, st));
     // `s` lives on this stack frame: the copy must have read it before return
     EDL_HIP(hipStreamSynchronize(st));
   }
-  cd.q0 = q0;
-  cd.q1 = q1;
-  cd.x = nullptr;
-  cd.ccoef = nullptr;
-  cd.counter = counter;
-  cd.sc = sc;
-  cd.alpha = alpha;
-  cd.beta = beta;
-  cd.nmax = nmax;
-  cd.brk_tol = 1e-14;
 }
 
 // Autotuned schedule cache: key = (precision, sum of dims, #chains).
@@ -2587,57 +2592,89 @@ static int64_t tridiag_group(Ctx& c, const std::vector<SeedSpec>& seeds, const s
     }
     if (alone) bt = false;
   }
-  // every buffer of the group in one allocation
-  Arena ar;
+  // every vector of the group in one allocation, and every chain's scalars and
+  // coefficients in another, which one copy brings back
+  Arena ar, small;
   {
-    size_t bytes = 0;
+    size_t bytes = 0, sbytes = 0;
     for (size_t k = 0; k < idx.size(); ++k) {
       const Sector& J = get_sector(c, targets[idx[k]]);
       const int ld = (bt || alone) ? padded_ld(J.sp[0].dim) : J.sp[0].dim;
       const int64_t D = (int64_t)ld * J.sp[1].dim;
-      bytes += ChainAlloc<T>::arena_bytes(D, (int)std::min<int64_t>(nlanc, J.dim));
+      bytes += ChainAlloc<T>::vector_bytes(D);
+      sbytes += ChainAlloc<T>::small_bytes((int)std::min<int64_t>(nlanc, J.dim));
       if (bt)
         bytes += Arena::round(sizeof(T) * D) + Arena::round(sizeof(double) * J.sp[0].dim) +
                  Arena::round(sizeof(double) * J.sp[1].dim);
     }
     ar.reserve(bytes);
+    small.reserve(sbytes);
   }
-  // Seeds are generated one after another into tmp (stream order keeps the
-  // reuse safe); their norms stay on the device until every chain is set up.
+  // The operator seeds of a batched group are built by one launch
+  // (launch_seed_group).  Any other seed is generated into tmp, one after another
+  // (stream order keeps the reuse safe); their norms stay on the device until
+  // every chain is set up.
+  auto grouped = [&](size_t k) { return bt && !host_seed && seeds[idx[k]].op != EDL_OP_J; };
   // The partial sums serve the seed norm (J.dim elements) and the stored
   // start vector's sum of squares (ld * DimDw elements, ld >= DimUp rounded
   // up to 32 rows: up to 32x J.dim on sectors with one up string).
-  DevBuf tmp(sizeof(double) * maxdim);
   const size_t nc = idx.size();
-  int64_t maxred = std::max<int64_t>(maxdim, 1);
+  size_t ng = 0;
+  for (size_t k = 0; k < nc; ++k) ng += grouped(k) ? 1 : 0;
+  DevBuf tmp(ng < nc ? sizeof(double) * maxdim : 0);
+  int64_t maxred = 1;
   for (size_t k = 0; k < idx.size(); ++k) {
+    if (grouped(k)) continue;
     const Sector& J = get_sector(c, targets[idx[k]]);
     const int ld = (bt || alone) ? padded_ld(J.sp[0].dim) : J.sp[0].dim;
-    maxred = std::max<int64_t>(maxred, (int64_t)ld * J.sp[1].dim);
+    maxred = std::max<int64_t>(maxred, std::max<int64_t>(maxdim, (int64_t)ld * J.sp[1].dim));
   }
   const int64_t part_n = partials_size(maxred);
   DevBuf sums(sizeof(double) * 2 * nc), part(sizeof(double) * (size_t)part_n);
   double* d_n2 = sums.as<double>();
   double* d_ss = d_n2 + nc;
+  std::vector<SeedChain> group;
+  std::vector<LzScalars*> scp;  // the scalars of the other chains
   for (size_t k = 0; k < nc; ++k) {
     const int s = idx[k];
     Sector& J = get_sector(c, targets[s]);
-    if (host_seed) {
-      EDL_HIP(hipMemcpyAsync(tmp.p, host_seed, sizeof(double) * J.dim, hipMemcpyHostToDevice, st));
-    } else {
-      const Sector& I = gs_sector_of(c, "edl_tridiag_batched");
-      if (seeds[s].op == EDL_OP_J)
-        launch_current_seed(current_terms(c.model, seeds[s].io), c.d_gs, J, tmp.as<double>(), st);
-      else
-        launch_seed(seeds[s], c.d_gs, I.sp[0].dim, J, tmp.as<double>(), st);
-    }
-    EDL_CHECK(partials_size(J.dim) <= part_n, "tridiag_group: partial-sum buffer smaller than the launch grid");
-    device_dot_to(tmp.as<double>(), tmp.as<double>(), J.dim, part.as<double>(), d_n2 + k, st);
     const int nmax = (int)std::min<int64_t>(nlanc, J.dim);
     ChainDev cd{};
     const int ld = (bt || alone) ? padded_ld(J.sp[0].dim) : J.sp[0].dim;
     allocs[k].ar = &ar;
-    init_chain<T>(c, cd, allocs[k], J, tmp.as<double>(), 0.0, nmax, st, ld, d_ss + k, part.as<double>(), part_n);
+    allocs[k].small = &small;
+    if (grouped(k)) {
+      place_chain(cd, allocs[k], J, nmax, ld);
+      SeedChain g{};
+      g.seed = seeds[s];
+      g.map_up = J.sp[0].map;
+      g.map_dw = J.sp[1].map;
+      g.dimup = J.sp[0].dim;
+      g.dimdw = J.sp[1].dim;
+      g.ld = ld;
+      g.nmax = nmax;
+      g.q0 = cd.q0;
+      g.q1 = cd.q1;
+      g.sc = cd.sc;
+      g.alpha = cd.alpha;
+      g.beta = cd.beta;
+      group.push_back(g);
+    } else {
+      if (host_seed) {
+        EDL_HIP(hipMemcpyAsync(tmp.p, host_seed, sizeof(double) * J.dim, hipMemcpyHostToDevice, st));
+      } else {
+        const Sector& I = gs_sector_of(c, "edl_tridiag_batched");
+        if (seeds[s].op == EDL_OP_J)
+          launch_current_seed(current_terms(c.model, seeds[s].io), c.d_gs, J, tmp.as<double>(), st);
+        else
+          launch_seed(seeds[s], c.d_gs, I.sp[0].dim, J, tmp.as<double>(), st);
+      }
+      EDL_CHECK(partials_size(J.dim) <= part_n, "tridiag_group: partial-sum buffer smaller than the launch grid");
+      const size_t o = scp.size();
+      device_dot_to(tmp.as<double>(), tmp.as<double>(), J.dim, part.as<double>(), d_n2 + o, st);
+      init_chain<T>(c, cd, allocs[k], J, tmp.as<double>(), 0.0, nmax, st, ld, d_ss + o, part.as<double>(), part_n);
+      scp.push_back(cd.sc);
+    }
     if (bt) {
       BtChain b{};
       b.V = two_pass_view(J, ld);
@@ -2661,15 +2698,19 @@ static int64_t tridiag_group(Ctx& c, const std::vector<SeedSpec>& seeds, const s
   }
   if (chains.empty()) return 0;
   {
-    std::vector<LzScalars*> scp(nc);
-    for (size_t k = 0; k < nc; ++k) scp[k] = chains[k].sc;
-    DevBuf d_scp(sizeof(LzScalars*) * nc);
-    EDL_HIP(hipMemcpyAsync(d_scp.p, scp.data(), sizeof(LzScalars*) * nc, hipMemcpyHostToDevice, st));
-    launch_init_scalars(d_scp.as<LzScalars*>(), d_n2, d_ss, (int)nc, st);
-    std::vector<double> n2h(nc);
-    EDL_HIP(hipMemcpyAsync(n2h.data(), d_n2, sizeof(double) * nc, hipMemcpyDeviceToHost, st));
+    // (the descriptors and the seeds' buffers are waited for before they go)
+    const size_t gpart = seed_group_blocks(group);
+    DevBuf d_scp(sizeof(LzScalars*) * scp.size()), d_group(sizeof(SeedChain) * group.size()),
+        d_gpart(2 * sizeof(double) * gpart);
+    if (!group.empty()) {
+      const Sector& I = gs_sector_of(c, "edl_tridiag_batched");
+      launch_seed_group<T>(group, d_group.as<SeedChain>(), d_gpart.as<double>(), c.d_gs, I.sp[0].dim, st);
+    }
+    if (!scp.empty()) {
+      EDL_HIP(hipMemcpyAsync(d_scp.p, scp.data(), sizeof(LzScalars*) * scp.size(), hipMemcpyHostToDevice, st));
+      launch_init_scalars(d_scp.as<LzScalars*>(), d_n2, d_ss, (int)scp.size(), st);
+    }
     EDL_HIP(hipStreamSynchronize(st));
-    for (size_t k = 0; k < nc; ++k) norm2[which[k]] = n2h[k];
   }
   const int steps = *std::max_element(nmaxs.begin(), nmaxs.end());
   ChainSet<T> cs;
@@ -2746,29 +2787,26 @@ static int64_t tridiag_group(Ctx& c, const std::vector<SeedSpec>& seeds, const s
                  chains.size(), bt ? (persist ? "persistent two-pass" : "two-pass tile") : (alone ? "one-chain two-pass" : "single-pass"), bt ? shp.C : 0,
                  bt ? shp.RS : 0, nstreams, nstreams > 1 ? "s" : "", steps, ms, 1e3 * ms / steps);
   }
-  // every chain's scalars and coefficients requested, then one wait
-  std::vector<ChainOut> outs(chains.size());
-  std::vector<LzScalars> scs(chains.size());
-  for (size_t k = 0; k < chains.size(); ++k) {
-    outs[k].alpha.assign(nmaxs[k], 0.0);
-    outs[k].beta.assign(nmaxs[k], 0.0);
-    EDL_HIP(hipMemcpyAsync(&scs[k], cs.h[k].sc, sizeof(LzScalars), hipMemcpyDeviceToHost, st));
-    EDL_HIP(hipMemcpyAsync(outs[k].alpha.data(), cs.h[k].alpha, sizeof(double) * nmaxs[k], hipMemcpyDeviceToHost, st));
-    EDL_HIP(hipMemcpyAsync(outs[k].beta.data(), cs.h[k].beta, sizeof(double) * nmaxs[k], hipMemcpyDeviceToHost, st));
-  }
+  // every chain's scalars and coefficients in one copy
+  std::vector<char> out(small.off);
+  EDL_HIP(hipMemcpyAsync(out.data(), small.buf.p, out.size(), hipMemcpyDeviceToHost, st));
   EDL_HIP(hipStreamSynchronize(st));
+  const char* base = static_cast<const char*>(small.buf.p);
+  auto host_of = [&](const void* p) { return out.data() + (static_cast<const char*>(p) - base); };
   int64_t hxv = 0;
   for (size_t k = 0; k < chains.size(); ++k) {
-    ChainOut& o = outs[k];
-    o.nsteps = scs[k].nsteps;
-    o.norm2 = scs[k].norm2;
+    LzScalars sc;
+    std::memcpy(&sc, host_of(chains[k].sc), sizeof(sc));
+    const double* a = reinterpret_cast<const double*>(host_of(chains[k].alpha));
+    const double* b = reinterpret_cast<const double*>(host_of(chains[k].beta));
     const int s = which[k];
     for (int j = 0; j < nlanc; ++j) {
-      alpha[(size_t)s * nlanc + j] = j < nmaxs[k] ? o.alpha[j] : 0.0;
-      beta[(size_t)s * nlanc + j] = j < nmaxs[k] ? o.beta[j] : 0.0;
+      alpha[(size_t)s * nlanc + j] = j < nmaxs[k] ? a[j] : 0.0;
+      beta[(size_t)s * nlanc + j] = j < nmaxs[k] ? b[j] : 0.0;
     }
-    if (nsteps) nsteps[s] = o.nsteps;
-    hxv += o.nsteps;
+    norm2[s] = sc.norm2;
+    if (nsteps) nsteps[s] = sc.nsteps;
+    hxv += sc.nsteps;
   }
   return hxv;
 }

@@ -11,6 +11,28 @@ struct SeedSpec {
 
 void launch_seed(const SeedSpec& s, const double* gs, int gs_dimup, const Sector& target, double* out, hipStream_t st);
 
+// The start of one batched chain: its seed, and where its vectors (column stride
+// ld, q0 the seed in the chain's precision, q1 and the padding rows zero),
+// scalars and coefficients go.  blocks and part are set by launch_seed_group.
+struct LzScalars;
+struct SeedChain {
+  SeedSpec seed;
+  const int32_t* map_up;
+  const int32_t* map_dw;
+  int dimup, dimdw, ld, nmax, blocks;
+  void *q0, *q1;
+  LzScalars* sc;
+  double *alpha, *beta;  // [nmax], zeroed
+  double* part;          // [2 * blocks] sums of the seed's and the stored vector's squares
+};
+// Sets every chain's block count; returns their sum (d_part holds twice as many doubles).
+size_t seed_group_blocks(std::vector<SeedChain>& g);
+// Every chain of g built, summed and its scalars set, in two launches.  `g` is
+// copied to d_g and has to live until the stream is waited for.
+template <typename T>
+void launch_seed_group(std::vector<SeedChain>& g, SeedChain* d_g, double* d_part, const double* gs, int gs_dimup,
+                       hipStream_t st);
+
 // Current-operator seed of the optical conductivity of one orbital
 // (lanc_ed_build_oc, OC_ELECTRONS.f90:103-213): terms coef * c+_a c_b of one
 // spin along the ring order of the orbital's sites, in the ground-state
