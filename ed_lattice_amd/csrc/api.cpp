@@ -2297,9 +2297,13 @@ static std::vector<BtChain> bt_resized(std::vector<BtChain> v, const BtShape& s)
 template <typename T>
 static BtShape bt_tune(Ctx& c, const std::vector<BtChain>& chains, int max_up, int max_dw, hipStream_t st) {
   const char* fk = std::getenv("EDL_BATCHED_UP_H16");
+  // EDL_BATCHED_SLAB_ROWS keeps the tuner to one slab height
+  const char* fr = std::getenv("EDL_BATCHED_SLAB_ROWS");
+  const int rs_only = fr ? std::atoi(fr) : 0;
+  EDL_CHECK(rs_only >= 0 && rs_only <= 32 && (rs_only & (rs_only - 1)) == 0, "EDL_BATCHED_SLAB_ROWS must be 1, 2, 4 .. 32");
   const int forms = (bt_h16_ok(chains, 0) ? 1 : 0) + (bt_h16_ok(chains, 1) ? 2 : 0);  // two-hop tables of each spin
   const auto key = std::make_tuple((int)sizeof(T), max_up, max_dw, (int)chains.size(),
-                                   4 * (fk ? std::atoi(fk) + 1 : 0) + forms);
+                                   4 * (fk ? std::atoi(fk) + 1 : 0) + forms + 64 * rs_only);
   auto it = bt_cache().find(key);
   if (it != bt_cache().end()) return it->second;
   BtShape best = bt_shape(max_up, max_dw, sizeof(T));
@@ -2370,6 +2374,7 @@ static BtShape bt_tune(Ctx& c, const std::vector<BtChain>& chains, int max_up, i
   for (int h16 : {0, 1}) {
     if ((h16 && !h16_dw_ok) || (h16_only >= 0 && h16 != h16_only)) continue;
     for (int RS : {32, 16, 8, 4, 2, 1}) {
+      if (rs_only && RS != rs_only) continue;
       if ((size_t)RS * sizeof(T) > 128 || bt_dw_lds_bytes(max_dw, RS, sizeof(T), h16) > budget) continue;
       for (int nc : {1, 2})
         for (int th : {256, 512, 1024}) {
@@ -2379,6 +2384,9 @@ static BtShape bt_tune(Ctx& c, const std::vector<BtChain>& chains, int max_up, i
           w.threads_dw = th;
           w.dw_h16 = h16;
           const double ms = time(w, false);
+          if (verbose())
+            std::fprintf(stderr, "[edl] tune tiles down fp%d RS %2d nc %d%s x %4d: %.4f ms\n", 8 * (int)sizeof(T), RS,
+                         nc, h16 ? " two-hop" : "", th, ms);
           if (ms < bd) {
             bd = ms;
             best.RS = RS;

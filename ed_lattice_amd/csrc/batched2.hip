@@ -263,9 +263,131 @@ static __device__ __forceinline__ double bt_dw_slab(const TwoPassView& V, const 
   return part;
 }
 
+// The same slab with 16 bytes of consecutive rows a lane (Row16: 4 in fp32, 2 in
+// fp64): a hop word, its coefficient and its address serve VW rows, and every
+// global and LDS access is 16 bytes.  RS is a multiple of VW and V.ld of 32, so
+// that a slab's rows past dimup are the column's padding: zero in q and q_{k-1},
+// unwritten in T, and zero again in t.  Each row's sum runs in the order of the
+// one-row form.  With a row a lane the tile was bound by what each hop cost a lane
+// (word, coefficient, address, LDS issue), not by memory: 3x4, 12 fp32 chains of
+// several hopping values 77 -> 38 us a launch, 156 fp64 chains 1006 -> 835 us
+// (2.9 -> 3.5 TB/s of its 2.9 GB).  The faster of the two at every slab height and
+// block size that both have.
+template <typename T, int RS, int SB>
+static __device__ __forceinline__ void bt_stage_slab_v(const TwoPassView& V, T* S, const T* __restrict__ q, int r0) {
+  typedef typename Row16<T>::type VT;
+  constexpr int VW = 16 / (int)sizeof(T), LPS = RS / VW;
+  const int n = V.dimdw * LPS;
+  const size_t ld = (size_t)V.ld;
+  VT* Sv = reinterpret_cast<VT*>(S);
+  for (int base = 0; base < n; base += SB * (int)blockDim.x) {
+    VT a[SB];
+#pragma unroll
+    for (int h = 0; h < SB; ++h) {
+      const int i = min(base + h * (int)blockDim.x + (int)threadIdx.x, n - 1);
+      a[h] = *reinterpret_cast<const VT*>(q + (size_t)(i / LPS) * ld + r0 + (i % LPS) * VW);
+    }
+#pragma unroll
+    for (int h = 0; h < SB; ++h) {
+      const int i = base + h * (int)blockDim.x + (int)threadIdx.x;
+      if (i < n) Sv[i] = a[h];
+    }
+  }
+}
+template <typename T, int RS, int NC, bool H16>
+static __device__ __forceinline__ double bt_dw_slab_v(const TwoPassView& V, const T* lut, const T* S, const int* cntS,
+                                                      T* __restrict__ qo, const T* __restrict__ tb, int r0, T ts,
+                                                      T bo) {
+  typedef typename Row16<T>::type VT;
+  constexpr int VW = 16 / (int)sizeof(T), LPS = RS / VW, KCH = 8;
+  const int dimdw = V.dimdw;
+  const size_t ld = (size_t)V.ld;
+  const VT* Sv = reinterpret_cast<const VT*>(S);
+  const int rv = threadIdx.x % LPS, jl = threadIdx.x / LPS, jstep = blockDim.x / LPS;
+  const int row = r0 + rv * VW, live = V.dimup - row;  // rows of this lane that exist
+  const T l0 = H16 ? lut[0] : (T)0;
+  double part = 0.0;
+  for (int j0 = jl; j0 < dimdw; j0 += NC * jstep) {
+    int col[NC], nh[NC], nmax = 0;
+    bool okc[NC];
+    size_t ii[NC];
+    VT tin[NC], qold[NC], acc[NC];
+#pragma unroll
+    for (int h = 0; h < NC; ++h) {
+      col[h] = j0 + h * jstep;
+      okc[h] = col[h] < dimdw;
+      if (!okc[h]) col[h] = j0;
+      nh[h] = okc[h] ? (H16 ? (cntS[col[h]] + 1) >> 1 : cntS[col[h]]) : 0;
+      nmax = nh[h] > nmax ? nh[h] : nmax;
+      ii[h] = (size_t)col[h] * ld + row;
+      tin[h] = *reinterpret_cast<const VT*>(tb + ii[h]);
+      qold[h] = *reinterpret_cast<const VT*>(qo + ii[h]);
+#pragma unroll
+      for (int e = 0; e < VW; ++e) acc[h][e] = (T)0;
+    }
+    if constexpr (H16) {
+      constexpr int KW = KCH / 2;  // words (two hops each) per chunk
+      const uint32_t zpad = (uint32_t)dimdw | ((uint32_t)dimdw << 16);
+      for (int k0 = 0; k0 < nmax; k0 += KW) {
+        uint32_t w[NC][KW];
+#pragma unroll
+        for (int h = 0; h < NC; ++h)
+#pragma unroll
+          for (int jj = 0; jj < KW; ++jj)
+            w[h][jj] = (k0 + jj < nh[h]) ? V.pk16_dw[(size_t)(k0 + jj) * dimdw + col[h]] : zpad;
+#pragma unroll
+        for (int h = 0; h < NC; ++h)
+#pragma unroll
+          for (int jj = 0; jj < KW; ++jj) {
+            const uint32_t wl = w[h][jj];
+            const T cl = flip_sign(l0, (wl << 16) & 0x80000000u), ch = flip_sign(l0, wl & 0x80000000u);
+            const VT xl = Sv[(int)(wl & 0x7FFFu) * LPS + rv], xh = Sv[(int)((wl >> 16) & 0x7FFFu) * LPS + rv];
+#pragma unroll
+            for (int e = 0; e < VW; ++e) {
+              acc[h][e] += cl * xl[e];
+              acc[h][e] += ch * xh[e];
+            }
+          }
+      }
+    } else {
+      for (int k0 = 0; k0 < nmax; k0 += KCH) {
+        uint32_t w[NC][KCH];
+#pragma unroll
+        for (int h = 0; h < NC; ++h)
+#pragma unroll
+          for (int jj = 0; jj < KCH; ++jj)
+            w[h][jj] = (k0 + jj < nh[h]) ? V.pk_dw[(size_t)(k0 + jj) * dimdw + col[h]] : (255u << 24);
+#pragma unroll
+        for (int h = 0; h < NC; ++h)
+#pragma unroll
+          for (int jj = 0; jj < KCH; ++jj) {
+            const T cf = lut[w[h][jj] >> 24];
+            const VT x = Sv[(int)(w[h][jj] & 0xFFFFFFu) * LPS + rv];
+#pragma unroll
+            for (int e = 0; e < VW; ++e) acc[h][e] += cf * x[e];
+          }
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < NC; ++h) {
+      if (!okc[h]) continue;
+      const VT self = Sv[col[h] * LPS + rv];
+      VT tv;
+#pragma unroll
+      for (int e = 0; e < VW; ++e) {
+        tv[e] = e < live ? (tin[h][e] + acc[h][e]) * ts - bo * qold[h][e] : (T)0;
+        part += (double)tv[e] * (double)self[e];
+      }
+      *reinterpret_cast<VT*>(qo + ii[h]) = tv;
+    }
+  }
+  return part;
+}
+
 template <typename T, int RS, int NC, bool H16 = false>
 __global__ __launch_bounds__(1024) void k_bt_dw(const BtChain* __restrict__ chains, const int64_t* __restrict__ tile0,
                                                 const int32_t* __restrict__ tchain, int64_t Tall, int64_t n8) {
+  constexpr bool VEC = bt_dw_vec_rows(RS, sizeof(T));
   extern __shared__ __align__(16) unsigned char smem[];
   T* lut = reinterpret_cast<T*>(smem);
   T* S = reinterpret_cast<T*>(smem + lds_head_bytes(sizeof(T)));  // [dimdw][RS]
@@ -288,7 +410,10 @@ __global__ __launch_bounds__(1024) void k_bt_dw(const BtChain* __restrict__ chai
   // together and written to LDS after (one memory round trip, not three)
   const T lv = (!H16 && threadIdx.x < 256) ? lsrc[threadIdx.x] : (T)0;
   const int cv = (int)threadIdx.x < V.dimdw ? V.cnt_dw[threadIdx.x] : 0;
-  bt_stage_slab<T, RS>(V, S, q, sl * RS);
+  if constexpr (VEC)
+    bt_stage_slab_v<T, RS, 4>(V, S, q, sl * RS);
+  else
+    bt_stage_slab<T, RS>(V, S, q, sl * RS);
   if (H16) {
     if (threadIdx.x < RS) S[(size_t)V.dimdw * RS + threadIdx.x] = (T)0;
   } else {
@@ -300,7 +425,11 @@ __global__ __launch_bounds__(1024) void k_bt_dw(const BtChain* __restrict__ chai
   __syncthreads();
   const double inv_s = 1.0 / s.s_cur;
   const T ts = (T)inv_s, bo = (T)(s.beta_k / s.s_old);
-  const double part = bt_dw_slab<T, RS, NC, false, H16>(V, H16 ? lsrc : lut, S, cntS, q, qo, tb, sl * RS, ts, bo);
+  double part;
+  if constexpr (VEC)
+    part = bt_dw_slab_v<T, RS, NC, H16>(V, H16 ? lsrc : lut, S, cntS, qo, tb, sl * RS, ts, bo);
+  else
+    part = bt_dw_slab<T, RS, NC, false, H16>(V, H16 ? lsrc : lut, S, cntS, q, qo, tb, sl * RS, ts, bo);
   const double v = block_sum(part * inv_s, sh);
   if (threadIdx.x == 0) B.partD[sl] = v;
 }
@@ -556,6 +685,7 @@ static void bt_dw_r(const BtSet& bs, hipStream_t st, bool scalars) {
   EDL_CHECK(bs.shape.threads_dw % RS == 0, "bt_launch_dw: block size not a multiple of the slab height");
   EDL_CHECK(!h16 || bt_h16_ok(bs.h, 1), "bt_launch_dw: a chain's sector has no two-hop table");
   const int64_t n8 = (bs.tiles_dw + 7) / 8;
+  for (const BtChain& b : bs.h) EDL_CHECK(b.V.ld % 32 == 0, "bt_launch_dw: column stride not padded");
   if (h16)
     hipLaunchKernelGGL((k_bt_dw<T, RS, NC, true>), dim3((unsigned)(8 * n8)), dim3(bs.shape.threads_dw), lds, st,
                        bs.d, bs.d_tile_dw, bs.d_chain_dw, bs.tiles_dw, n8);

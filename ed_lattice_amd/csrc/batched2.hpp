@@ -47,6 +47,9 @@ struct BtShape {
   int up_h16 = 0;        // 1: the up tiles read the hops two to a word (bt_h16_ok, spin 0)
   int dw_h16 = 0;        // 1: the down tiles likewise (spin 1)
 };
+// Slabs of at least 16 bytes a column take 16 bytes of rows a lane in the down
+// tiles; lower ones (columns of more than about 9 000 strings) one row a lane.
+constexpr bool bt_dw_vec_rows(int RS, size_t elem) { return RS * elem >= 16; }
 
 // Largest up panel width and down slab height that fit the sectors, or
 // RS = 0 when some sector does not fit (the caller then takes the
