@@ -1014,8 +1014,9 @@ __global__ __launch_bounds__(256) void k_lz_beta(LzChain L, int nparts) {
   }
 }
 
-// After the down pass: alpha_k; phase B of step k becomes pending.
-__global__ __launch_bounds__(256) void k_lz_alpha(LzChain L, int nparts) {
+// After the down pass: alpha_k; phase B of step k becomes pending.  The order of
+// the sum follows the block size (launch_lz_alpha).
+__global__ __launch_bounds__(1024) void k_lz_alpha(LzChain L, int nparts) {
   __shared__ double sh[16];
   const LzScalars s = *L.sc;
   if (s.stopped) return;
@@ -1726,7 +1727,11 @@ void launch_lz_beta(const LzChain& L, const TwoPassView& V, const TwoPassCfg& cf
 }
 
 void launch_lz_alpha(const LzChain& L, const TwoPassView& V, const TwoPassCfg& cfg, hipStream_t st) {
-  hipLaunchKernelGGL(k_lz_alpha, dim3(1), dim3(256), 0, st, L, pass_dw_grid(V, cfg));
+  // Two-launch steps: as many threads as the up pass, whose blocks add the same
+  // partials up (block_sum_of), so that alpha_k has the same bits whether this
+  // launch takes it (a checked step, the last one) or the next up pass.
+  const int threads = L.sc2 ? cfg.threads_up : 256;
+  hipLaunchKernelGGL(k_lz_alpha, dim3(1), dim3(threads), 0, st, L, pass_dw_grid(V, cfg));
   EDL_HIP(hipGetLastError());
 }
 
