@@ -1918,10 +1918,59 @@ extern "C" int edl_hxv(edl_ctx* ctx, int isector, int prec, const void* v, void*
   API_END
 }
 
-// edl_hxv_noalloc: the two passes with the intermediate T in the file-scope
-// device scratch, the schedule the tuner cached for this sector shape (a
-// fixed one when none is cached: tuning allocates), no allocation, no
-// events.
+// The operator's schedule where nothing may be allocated, so nothing tuned: what
+// is cached for the column stride, else for the engine's padded stride (host
+// products), else the chain's shapes (ground states and seeds tune only those),
+// else a fixed one.  Shapes of the padded stride serve the natural one: 3x4 fp64
+// after a host product @A us a call against @B us on the fixed two passes, after a
+// ground state @C us, 3x5 (7,4) fp32 after a ground state @D against 182 us.  Of the
+// fixed ones, sectors of the one-launch form's size take that, a column a block:
+// resident ground states tune nothing (8-ring fp64 @E against 21.2 us).
+template <typename T>
+static TwoPassCfg untuned_cfg(Ctx& c, const Sector& s, int ld) {
+  const SpinTable &u = s.sp[0], &d = s.sp[1];
+  const char* from = nullptr;
+  TwoPassCfg cfg;
+  for (int l : {ld, padded_ld(u.dim)}) {
+    auto it = tp_cache().find({u.dim, d.dim, hop_key(s, 0), hop_key(s, 1), l, one_pass_key(sizeof(T))});
+    if (it == tp_cache().end()) continue;
+    cfg = it->second;
+    from = l == ld ? "this stride" : "the padded stride";
+    break;
+  }
+  if (!from) {
+    auto it = tp_chain_cache().find({u.dim, d.dim, hop_key(s, 0), hop_key(s, 1), (int)sizeof(T)});
+    if (it != tp_chain_cache().end()) {
+      cfg = chain_cfg(it->second);
+      from = "the chain";
+    }
+  }
+  if (!from) {
+    from = "none, two passes";
+    cfg.C = 1;
+    cfg.up_rpt = 2;
+    cfg.up_kch = 8;
+    cfg.threads_up = 1024;
+    cfg.grid_up = c.num_cu;
+    cfg.R = 64;
+    cfg.threads_dw = 256;
+    cfg.nchunk = std::min(32, d.dim);
+    cfg.ncol = 1;
+    cfg.kch = 16;
+    cfg.dw_vec = 0;
+    if (one_pass_size(s, sizeof(T)) && cols_ok(two_pass_view(s, ld), 1, sizeof(T))) {
+      from = "none, one launch";
+      cfg.one_C = 1;
+      cfg.one_threads = std::min(1024, (u.dim + 63) / 64 * 64);
+    }
+  }
+  if (verbose()) std::fprintf(stderr, "[edl] noalloc schedule tuned for: %s\n", from);
+  return cfg;
+}
+
+// edl_hxv_noalloc: the operator with the two passes' intermediate T in the
+// file-scope device scratch, a schedule that is there (untuned_cfg), no
+// allocation, no events.
 template <typename T>
 static void hxv_noalloc_impl(Ctx& c, Sector& s, const T* v, T* hv) {
   EDL_CHECK(!seg_path(s, sizeof(T)) && two_pass_ok(s, sizeof(T)),
@@ -1931,24 +1980,7 @@ static void hxv_noalloc_impl(Ctx& c, Sector& s, const T* v, T* hv) {
   EDL_CHECK(bytes <= noalloc_scratch_bytes(),
             "edl_hxv_noalloc: the sector's intermediate (" + std::to_string(bytes) +
                 " bytes) exceeds the 256 MiB scratch; use edl_hxv");
-  const auto key = std::make_tuple(s.sp[0].dim, s.sp[1].dim, hop_key(s, 0), hop_key(s, 1), ld, one_pass_key(sizeof(T)));
-  TwoPassCfg cfg;
-  auto it = tp_cache().find(key);
-  if (it != tp_cache().end()) {
-    cfg = it->second;
-  } else {
-    cfg.C = 1;
-    cfg.up_rpt = 2;
-    cfg.up_kch = 8;
-    cfg.threads_up = 1024;
-    cfg.grid_up = c.num_cu;
-    cfg.R = 64;
-    cfg.threads_dw = 256;
-    cfg.nchunk = std::min(32, s.sp[1].dim);
-    cfg.ncol = 1;
-    cfg.kch = 16;
-    cfg.dw_vec = 0;
-  }
+  const TwoPassCfg cfg = untuned_cfg<T>(c, s, ld);
   const TwoPassView V = two_pass_view(s, ld);
   T* tmp = static_cast<T*>(noalloc_scratch(c.device));
   T* vin = const_cast<T*>(v);  // operator mode only reads it
