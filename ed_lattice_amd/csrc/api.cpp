@@ -1922,10 +1922,11 @@ extern "C" int edl_hxv(edl_ctx* ctx, int isector, int prec, const void* v, void*
 // is cached for the column stride, else for the engine's padded stride (host
 // products), else the chain's shapes (ground states and seeds tune only those),
 // else a fixed one.  Shapes of the padded stride serve the natural one: 3x4 fp64
-// after a host product @A us a call against @B us on the fixed two passes, after a
-// ground state @C us, 3x5 (7,4) fp32 after a ground state @D against 182 us.  Of the
-// fixed ones, sectors of the one-launch form's size take that, a column a block:
-// resident ground states tune nothing (8-ring fp64 @E against 21.2 us).
+// after a host product 28.9 us a call and after a ground state 30.1, against 51.7
+// on the fixed two passes (28.0 tuned for the call itself); 3x5 (7,4) fp32 after a
+// ground state 95 us against 182 (86 tuned).  Of the fixed ones, sectors of the
+// one-launch form's size take that, a column a block: resident ground states tune
+// nothing (8-ring fp64 14.9 us against 21.2; 3x4 fp64 32.6).
 template <typename T>
 static TwoPassCfg untuned_cfg(Ctx& c, const Sector& s, int ld) {
   const SpinTable &u = s.sp[0], &d = s.sp[1];
