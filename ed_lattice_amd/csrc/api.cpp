@@ -57,84 +57,6 @@ static void release_sectors(Ctx& c) {
   c.sectors.clear();
 }
 
-// ------------------------------------------------------- device memory
-void* DevPool::take(size_t bytes) {
-  // sizes in steps of an eighth, so that buffers of nearly equal calls match
-  size_t step = 512;
-  while (step * 16 <= bytes) step *= 2;
-  const size_t want = (std::max<size_t>(bytes, 1) + step - 1) / step * step;
-  auto it = free_.lower_bound(want);
-  if (it != free_.end() && it->first <= want + want / 4) {
-    void* p = it->second;
-    cached_ -= it->first;
-    live_[p] = it->first;
-    free_.erase(it);
-    return p;
-  }
-  void* p = nullptr;
-  if (hipMalloc(&p, want) != hipSuccess) {
-    (void)hipGetLastError();
-    release();
-    if (hipMalloc(&p, want) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
-  }
-  live_[p] = want;
-  return p;
-}
-void DevPool::give(void* p) {
-  if (!p) return;
-  auto it = live_.find(p);
-  if (it == live_.end()) {
-    (void)hipFree(p);
-    return;
-  }
-  const size_t n = it->second;
-  live_.erase(it);
-  if (!bound_) {
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) (void)hipGetLastError();
-    bound_ = std::max<size_t>(total_b / 16, 1);
-  }
-  if (cached_ + n > bound_) {
-    (void)hipFree(p);
-    return;
-  }
-  free_.emplace(n, p);
-  cached_ += n;
-}
-void DevPool::release() {
-  for (auto& kv : free_) (void)hipFree(kv.second);
-  free_.clear();
-  cached_ = 0;
-}
-DevPool*& current_pool() {
-  static thread_local DevPool* p = nullptr;
-  return p;
-}
-void* dev_try_alloc(size_t bytes) {
-  if (DevPool* pool = current_pool()) return pool->take(bytes);
-  void* p = nullptr;
-  if (hipMalloc(&p, bytes ? bytes : 4) != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  return p;
-}
-void* dev_alloc(size_t bytes) {
-  void* p = dev_try_alloc(bytes);
-  if (!p) throw Error("out of device memory (" + std::to_string(bytes) + " bytes)");
-  return p;
-}
-void dev_free(void* p) {
-  if (!p) return;
-  if (DevPool* pool = current_pool())
-    pool->give(p);
-  else
-    (void)hipFree(p);
-}
-
 // ------------------------------------------------------------ utilities
 struct DevBuf {
   void* p = nullptr;
@@ -163,11 +85,11 @@ struct DevBuf {
   }
 };
 
-// Device memory a call can still take: free, or cached by its own context.
+// Device memory a call can still take: free, or cached by a context.
 static size_t available_bytes() {
   size_t free_b = 0, total_b = 0;
   EDL_HIP(hipMemGetInfo(&free_b, &total_b));
-  return free_b + (current_pool() ? current_pool()->cached() : 0);
+  return free_b + device_cached_bytes();
 }
 
 // Bump allocator over one device allocation: the buffers of a chain group
@@ -221,7 +143,7 @@ static void* scratch(Ctx& c, size_t bytes) {
     if (c.d_scratch) EDL_HIP(hipFree(c.d_scratch));
     c.d_scratch = nullptr;
     c.scratch_bytes = 0;
-    EDL_HIP(hipMalloc(&c.d_scratch, bytes));
+    EDL_HIP(device_malloc(&c.d_scratch, bytes));
     c.scratch_bytes = bytes;
   }
   return c.d_scratch;
@@ -2097,7 +2019,7 @@ extern "C" int edl_device_alloc(edl_ctx* ctx, int64_t bytes, void** dev_ptr) {
   EDL_CHECK(dev_ptr && bytes > 0, "edl_device_alloc: bad arguments");
   EDL_HIP(hipSetDevice(ctx->c.device));
   void* p = nullptr;
-  EDL_HIP(hipMalloc(&p, (size_t)bytes));
+  EDL_HIP(device_malloc(&p, (size_t)bytes));
   ctx->c.user_bufs.push_back(p);
   *dev_ptr = p;
   API_END

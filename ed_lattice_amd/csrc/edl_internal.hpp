@@ -11,6 +11,8 @@
 #include <string>
 #include <vector>
 
+#include "pool.hpp"
+
 namespace edl {
 
 constexpr int kMaxNs = 31;      // spin strings are held in 32-bit words
@@ -220,40 +222,12 @@ void init_binomials();
 // The launchers of hxv.hip / hxv2.hip / seeds.hip are declared in chains.hpp,
 // hxv2.hpp and seeds.hpp.
 
-// Device buffers of finished calls, kept by their context for its next ones
-// (a hipMalloc or hipFree of small buffers costs 5 to 10 us each and waits for
-// the device, a gigabyte that was in use before about 25 ms).  Bounded: at most
-// a sixteenth of the device's memory stays cached, the rest is freed at once; given back
-// when the context is destroyed, takes a model of another number of sites, or
-// an allocation of this library fails.  All work of a context is ordered on
-// its stream, so a buffer put back while launches that use it are queued is
-// safe to hand to later launches.
-class DevPool {
- public:
-  void* take(size_t bytes);       // nullptr when the device has no memory
-  void give(void* p);             // p from take of any pool, or from hipMalloc
-  void release();                 // frees what is cached
-  size_t cached() const { return cached_; }
-  ~DevPool() { release(); }
-
- private:
-  std::multimap<size_t, void*> free_;
-  std::map<void*, size_t> live_;
-  size_t cached_ = 0, bound_ = 0;
-};
-// The pool of the context whose call this thread is in (set by PoolScope),
-// null outside: dev_alloc and dev_free then are hipMalloc and hipFree.
-DevPool*& current_pool();
-struct PoolScope {
-  DevPool* before;
-  explicit PoolScope(DevPool& p) : before(current_pool()) { current_pool() = &p; }
-  ~PoolScope() { current_pool() = before; }
-  PoolScope(const PoolScope&) = delete;
-  PoolScope& operator=(const PoolScope&) = delete;
-};
-void* dev_try_alloc(size_t bytes);
-void* dev_alloc(size_t bytes);    // throws Error
-void dev_free(void* p);
+// dev_try_alloc (pool.hpp), or an Error.
+inline void* dev_alloc(size_t bytes) {
+  void* p = dev_try_alloc(bytes);
+  if (!p) throw Error("out of device memory (" + std::to_string(bytes) + " bytes)");
+  return p;
+}
 
 struct Ctx {
   int device = 0;

@@ -1305,23 +1305,23 @@ static void build_color_table(SpinTable& t, int W, hipStream_t st) {
       }
     }
   }
-  EDL_HIP(hipMalloc(&ct.words, sizeof(uint32_t) * std::max<size_t>(words.size(), 1)));
-  EDL_HIP(hipMalloc(&ct.off, sizeof(int32_t) * nb));
-  EDL_HIP(hipMalloc(&ct.ns, sizeof(int32_t) * nb));
+  EDL_HIP(device_malloc(&ct.words, sizeof(uint32_t) * std::max<size_t>(words.size(), 1)));
+  EDL_HIP(device_malloc(&ct.off, sizeof(int32_t) * nb));
+  EDL_HIP(device_malloc(&ct.ns, sizeof(int32_t) * nb));
   EDL_HIP(hipMemcpyAsync(ct.words, words.data(), sizeof(uint32_t) * words.size(), hipMemcpyHostToDevice, st));
   EDL_HIP(hipMemcpyAsync(ct.off, off.data(), sizeof(int32_t) * nb, hipMemcpyHostToDevice, st));
   EDL_HIP(hipMemcpyAsync(ct.ns, ns.data(), sizeof(int32_t) * nb, hipMemcpyHostToDevice, st));
   if (h16) {
-    EDL_HIP(hipMalloc(&ct.words16, sizeof(uint32_t) * std::max<size_t>(w16.size(), 1)));
-    EDL_HIP(hipMalloc(&ct.off16, sizeof(int32_t) * nb));
-    EDL_HIP(hipMalloc(&ct.ns16, sizeof(int32_t) * nb));
+    EDL_HIP(device_malloc(&ct.words16, sizeof(uint32_t) * std::max<size_t>(w16.size(), 1)));
+    EDL_HIP(device_malloc(&ct.off16, sizeof(int32_t) * nb));
+    EDL_HIP(device_malloc(&ct.ns16, sizeof(int32_t) * nb));
     EDL_HIP(hipMemcpyAsync(ct.words16, w16.data(), sizeof(uint32_t) * w16.size(), hipMemcpyHostToDevice, st));
     EDL_HIP(hipMemcpyAsync(ct.off16, off16.data(), sizeof(int32_t) * nb, hipMemcpyHostToDevice, st));
     EDL_HIP(hipMemcpyAsync(ct.ns16, ns16.data(), sizeof(int32_t) * nb, hipMemcpyHostToDevice, st));
-    EDL_HIP(hipMalloc(&ct.words16s, sizeof(uint32_t) * std::max<size_t>(w16s.size(), 1)));
-    EDL_HIP(hipMalloc(&ct.off16s, sizeof(int32_t) * nb));
-    EDL_HIP(hipMalloc(&ct.ns16s, sizeof(int32_t) * nb));
-    EDL_HIP(hipMalloc(&ct.np16s, sizeof(int32_t) * nb));
+    EDL_HIP(device_malloc(&ct.words16s, sizeof(uint32_t) * std::max<size_t>(w16s.size(), 1)));
+    EDL_HIP(device_malloc(&ct.off16s, sizeof(int32_t) * nb));
+    EDL_HIP(device_malloc(&ct.ns16s, sizeof(int32_t) * nb));
+    EDL_HIP(device_malloc(&ct.np16s, sizeof(int32_t) * nb));
     EDL_HIP(hipMemcpyAsync(ct.words16s, w16s.data(), sizeof(uint32_t) * w16s.size(), hipMemcpyHostToDevice, st));
     EDL_HIP(hipMemcpyAsync(ct.off16s, off16s.data(), sizeof(int32_t) * nb, hipMemcpyHostToDevice, st));
     EDL_HIP(hipMemcpyAsync(ct.ns16s, ns16s.data(), sizeof(int32_t) * nb, hipMemcpyHostToDevice, st));
@@ -1348,7 +1348,7 @@ static void build_pair_table(SpinTable& t, hipStream_t st) {
       uint32_t& o = w[(size_t)(k / 2) * dim + a];
       o = (k & 1) ? ((o & 0xFFFFu) | (half << 16)) : ((o & 0xFFFF0000u) | half);
     }
-  EDL_HIP(hipMalloc(&t.pk16, sizeof(uint32_t) * w.size()));
+  EDL_HIP(device_malloc(&t.pk16, sizeof(uint32_t) * w.size()));
   EDL_HIP(hipMemcpyAsync(t.pk16, w.data(), sizeof(uint32_t) * w.size(), hipMemcpyHostToDevice, st));
   EDL_HIP(hipStreamSynchronize(st));  // w must outlive the copy
 }
@@ -1409,10 +1409,10 @@ void build_dw_range_tables(Sector& s, hipStream_t st) {
       }
       nloc[j] = a - off[j];
     }
-    EDL_HIP(hipMalloc(&rt.lo, sizeof(int32_t) * (n + 1)));
-    EDL_HIP(hipMalloc(&rt.words, sizeof(uint32_t) * std::max<size_t>(words.size(), 1)));
-    EDL_HIP(hipMalloc(&rt.off, sizeof(int32_t) * (dim + 1)));
-    EDL_HIP(hipMalloc(&rt.nloc, sizeof(int32_t) * dim));
+    EDL_HIP(device_malloc(&rt.lo, sizeof(int32_t) * (n + 1)));
+    EDL_HIP(device_malloc(&rt.words, sizeof(uint32_t) * std::max<size_t>(words.size(), 1)));
+    EDL_HIP(device_malloc(&rt.off, sizeof(int32_t) * (dim + 1)));
+    EDL_HIP(device_malloc(&rt.nloc, sizeof(int32_t) * dim));
     EDL_HIP(hipMemcpyAsync(rt.lo, lo.data(), sizeof(int32_t) * (n + 1), hipMemcpyHostToDevice, st));
     EDL_HIP(hipMemcpyAsync(rt.words, words.data(), sizeof(uint32_t) * words.size(), hipMemcpyHostToDevice, st));
     EDL_HIP(hipMemcpyAsync(rt.off, off.data(), sizeof(int32_t) * (dim + 1), hipMemcpyHostToDevice, st));
@@ -1493,9 +1493,9 @@ void build_dw_order(Sector& s, hipStream_t st) {
   uint32_t* d_csro = nullptr;
   int32_t* d_offo = nullptr;
   try {
-    EDL_HIP(hipMalloc(&d_ord, sizeof(int32_t) * dim));
-    EDL_HIP(hipMalloc(&d_csro, sizeof(uint32_t) * std::max<size_t>(csro.size(), 1)));
-    EDL_HIP(hipMalloc(&d_offo, sizeof(int32_t) * (dim + 1)));
+    EDL_HIP(device_malloc(&d_ord, sizeof(int32_t) * dim));
+    EDL_HIP(device_malloc(&d_csro, sizeof(uint32_t) * std::max<size_t>(csro.size(), 1)));
+    EDL_HIP(device_malloc(&d_offo, sizeof(int32_t) * (dim + 1)));
     EDL_HIP(hipMemcpyAsync(d_ord, ord.data(), sizeof(int32_t) * dim, hipMemcpyHostToDevice, st));
     EDL_HIP(hipMemcpyAsync(d_csro, csro.data(), sizeof(uint32_t) * csro.size(), hipMemcpyHostToDevice, st));
     EDL_HIP(hipMemcpyAsync(d_offo, offo.data(), sizeof(int32_t) * (dim + 1), hipMemcpyHostToDevice, st));
@@ -2355,7 +2355,7 @@ const std::vector<int>& seg_bounds(Sector& s, size_t elem, int C) {
   b.push_back(t.dim);
   if (s.d_seg) (void)hipFree(s.d_seg);
   s.d_seg = nullptr;
-  EDL_HIP(hipMalloc(&s.d_seg, sizeof(int) * b.size()));
+  EDL_HIP(device_malloc(&s.d_seg, sizeof(int) * b.size()));
   EDL_HIP(hipMemcpy(s.d_seg, b.data(), sizeof(int) * b.size(), hipMemcpyHostToDevice));
   s.seg_h = b;
   s.seg_cap = cap;

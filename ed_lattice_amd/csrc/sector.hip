@@ -209,8 +209,8 @@ static void build_rank_hops(SpinTable& t, int Ns, const std::vector<HopPair>& pa
     const uint32_t c = s & (0u - s), rr = s + c;  // next string of the same popcount
     s = (((rr ^ s) >> 2) / c) | rr;
   }
-  EDL_HIP(hipMalloc(&r.rlo, sizeof(uint32_t) * r.nlo));
-  EDL_HIP(hipMalloc(&r.rhi, sizeof(uint32_t) * r.nhi));
+  EDL_HIP(device_malloc(&r.rlo, sizeof(uint32_t) * r.nlo));
+  EDL_HIP(device_malloc(&r.rhi, sizeof(uint32_t) * r.nhi));
   EDL_HIP(hipMemcpyAsync(r.rlo, lo.data(), sizeof(uint32_t) * r.nlo, hipMemcpyHostToDevice, st));
   EDL_HIP(hipMemcpyAsync(r.rhi, hi.data(), sizeof(uint32_t) * r.nhi, hipMemcpyHostToDevice, st));
   EDL_HIP(hipStreamSynchronize(st));  // lo, hi (host) must outlive the copies
@@ -224,7 +224,7 @@ static void build_spin(Ctx& c, const Model& M, SpinTable& t, int spin /*0 up, 1 
   double xh = 1.0;
   for (int i = 1; i <= t.N; i++) xh = xh * (double)(Ns + 1 - i) / (double)i;
   t.dim = (t.N == 0) ? 1 : (int)(xh + 0.5);
-  EDL_HIP(hipMalloc(&t.map, sizeof(int32_t) * t.dim));
+  EDL_HIP(device_malloc(&t.map, sizeof(int32_t) * t.dim));
   hipLaunchKernelGGL(k_unrank, dim3(blocks_for(t.dim)), dim3(kBlock), 0, st, t.map, t.dim, t.N, Ns);
   EDL_HIP(hipGetLastError());
 
@@ -248,9 +248,9 @@ static void build_spin(Ctx& c, const Model& M, SpinTable& t, int spin /*0 up, 1 
   HopPair* d_pairs = nullptr;
   int32_t* d_cnt = nullptr;
   const int np = (int)pairs.size();
-  EDL_HIP(hipMalloc(&d_pairs, sizeof(HopPair) * (np > 0 ? np : 1)));
+  EDL_HIP(device_malloc(&d_pairs, sizeof(HopPair) * (np > 0 ? np : 1)));
   if (np) EDL_HIP(hipMemcpyAsync(d_pairs, pairs.data(), sizeof(HopPair) * np, hipMemcpyHostToDevice, st));
-  EDL_HIP(hipMalloc(&d_cnt, sizeof(int32_t) * t.dim));
+  EDL_HIP(device_malloc(&d_cnt, sizeof(int32_t) * t.dim));
   hipLaunchKernelGGL(k_hop_count, dim3(blocks_for(t.dim)), dim3(kBlock), 0, st, t.map, t.dim, d_pairs, np, d_cnt);
   std::vector<int32_t> cnt(t.dim);
   EDL_HIP(hipMemcpyAsync(cnt.data(), d_cnt, sizeof(int32_t) * t.dim, hipMemcpyDeviceToHost, st));
@@ -259,20 +259,20 @@ static void build_spin(Ctx& c, const Model& M, SpinTable& t, int spin /*0 up, 1 
   for (int v : cnt) kmax = v > kmax ? v : kmax;
   t.kmax = kmax;
   size_t n = (size_t)(kmax > 0 ? kmax : 1) * t.dim;
-  EDL_HIP(hipMalloc(&t.nbr, sizeof(int32_t) * n));
-  EDL_HIP(hipMalloc(&t.coef64, sizeof(double) * n));
-  EDL_HIP(hipMalloc(&t.coef32, sizeof(float) * n));
+  EDL_HIP(device_malloc(&t.nbr, sizeof(int32_t) * n));
+  EDL_HIP(device_malloc(&t.coef64, sizeof(double) * n));
+  EDL_HIP(device_malloc(&t.coef32, sizeof(float) * n));
   t.packed_ok = (t.nvals <= 127) && (t.dim < (1 << 24));
   if (t.packed_ok) {
-    EDL_HIP(hipMalloc(&t.packed, sizeof(uint32_t) * n));
+    EDL_HIP(device_malloc(&t.packed, sizeof(uint32_t) * n));
     for (int k = 0; k < 256; ++k) t.lut64[k] = 0.0;
     for (int v = 0; v < t.nvals; ++v) {
       t.lut64[2 * v] = vals[v];
       t.lut64[2 * v + 1] = -vals[v];
     }
     for (int k = 0; k < 256; ++k) t.lut32[k] = (float)t.lut64[k];
-    EDL_HIP(hipMalloc(&t.d_lut64, sizeof(t.lut64)));
-    EDL_HIP(hipMalloc(&t.d_lut32, sizeof(t.lut32)));
+    EDL_HIP(device_malloc(&t.d_lut64, sizeof(t.lut64)));
+    EDL_HIP(device_malloc(&t.d_lut32, sizeof(t.lut32)));
     EDL_HIP(hipMemcpyAsync(t.d_lut64, t.lut64, sizeof(t.lut64), hipMemcpyHostToDevice, st));
     EDL_HIP(hipMemcpyAsync(t.d_lut32, t.lut32, sizeof(t.lut32), hipMemcpyHostToDevice, st));
   }
@@ -288,8 +288,8 @@ static void build_spin(Ctx& c, const Model& M, SpinTable& t, int spin /*0 up, 1 
     }
     EDL_CHECK(tot < ((int64_t)1 << 31), "build_sector: hop table exceeds 2^31 words");
     off[t.dim] = (int32_t)tot;
-    EDL_HIP(hipMalloc(&t.off, sizeof(int32_t) * ((size_t)t.dim + 1)));
-    EDL_HIP(hipMalloc(&t.csr, sizeof(uint32_t) * (size_t)(tot > 0 ? tot : 1)));
+    EDL_HIP(device_malloc(&t.off, sizeof(int32_t) * ((size_t)t.dim + 1)));
+    EDL_HIP(device_malloc(&t.csr, sizeof(uint32_t) * (size_t)(tot > 0 ? tot : 1)));
     EDL_HIP(hipMemcpyAsync(t.off, off.data(), sizeof(int32_t) * off.size(), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_ell_to_csr, dim3(blocks_for(t.dim)), dim3(kBlock), 0, st, t.packed, d_cnt, t.off, t.dim,
                        t.csr);
@@ -331,7 +331,7 @@ static void build_spin(Ctx& c, const Model& M, SpinTable& t, int spin /*0 up, 1 
     P.pj[k] = M.inter.pj[k];
   }
   P.ust_jh = M.Ust - M.Jh;
-  EDL_HIP(hipMalloc(&t.diag, sizeof(double) * t.dim));
+  EDL_HIP(device_malloc(&t.diag, sizeof(double) * t.dim));
   hipLaunchKernelGGL(k_diag, dim3(blocks_for(t.dim)), dim3(kBlock), 0, st, t.map, t.dim, P, t.diag);
   EDL_HIP(hipGetLastError());
   EDL_HIP(hipStreamSynchronize(st));
