@@ -379,94 +379,124 @@ static __device__ __forceinline__ double stage_panel(const TwoPassView& V, typen
   return nrm;
 }
 
-// Operator mode (chain = 0): T = [D + H_up] qa.  Chain mode: phase B of the
-// previous step where one is pending (r = t - alpha_k v_k over t, block
-// partial of |r|^2 into L.part_up, replay term x += c_k v_k), then
-// T = [D + H_up] q (unscaled; the down pass divides by s).  When the chain
-// has run its nmax steps only the replay term remains.
-template <typename T, int C, int RPT, int UKCH, bool LREG, bool COL, bool H16, bool SGN, int PFR = 0>
-static __device__ __forceinline__ void pass_up_body(const TwoPassView& V, const InterParams& I,
-                                                    const T* __restrict__ lut_up, T* qa, T* qb,
-                                                    T* __restrict__ tout, const LzChain& L, int chain) {
+// The panel of an up-pass block in LDS and its coefficient table.  H16 takes its
+// two coefficients from registers: no LDS table, and the panel starts at the
+// base of the dynamic LDS (small gather offsets fold into the LDS
+// instructions), with the zero rows that unused slots gather written after it
+// (the staging never writes them).
+template <typename T, int C, bool H16>
+static __device__ __forceinline__ typename Vec<T, C>::type* up_lds(const TwoPassView& V, const T* lut_up, T*& lut) {
   typedef typename Vec<T, C>::type VT;
   extern __shared__ __align__(16) unsigned char smem[];
-  // H16 takes its two coefficients from registers: no LDS table, and the
-  // panel starts at the base of the dynamic LDS (small gather offsets fold
-  // into the LDS instructions)
-  T* lut = H16 ? const_cast<T*>(lut_up) : reinterpret_cast<T*>(smem);
+  lut = H16 ? const_cast<T*>(lut_up) : reinterpret_cast<T*>(smem);
   VT* P = reinterpret_cast<VT*>(smem + (H16 ? 0 : lds_head_bytes(sizeof(T))));
-  __shared__ double sh[16];
-  const int npan = (V.dimdw + C - 1) / C;
   if (H16 && threadIdx.x < 32) {
-    // the zero rows that unused slots gather (the staging below never writes them)
     VT z;
 #pragma unroll
     for (int j = 0; j < C; ++j) Vec<T, C>::set(z, j, (T)0);
     P[V.dimup + threadIdx.x] = z;
   }
-  if (!chain) {
-    if (!H16)
-      for (int k = threadIdx.x; k < 256; k += blockDim.x) lut[k] = lut_up[k];
-    if constexpr (PFR > 0) {
-      // the block's first panel is staged as usual; each later one is
-      // loaded into registers (PanelPrefetch) before the barrier that ends
-      // the current panel and written to P after it
-      const int dimup = V.dimup;
-      int pan = blockIdx.x;
-      if (pan >= npan) return;
-      stage_plain<T, C>(V, P, qa, pan * C);
-      __syncthreads();
-      for (;;) {
-        const int nxt = pan + (int)gridDim.x;
-        up_rows<T, C, RPT, UKCH, LREG, COL, H16, SGN>(V, I, lut, P, tout, pan * C, (T)1);
-        if (nxt >= npan) break;
-        // the next panel's loads go out as soon as this thread's rows are
-        // done, so their round trip overlaps the other waves' last rows and
-        // the barrier (the waves of a block end an iteration apart)
-        PanelPrefetch<T, C, PFR> pf;
-        const int c1 = nxt * C;
+  return P;
+}
+
+// Operator: T = [D + H_up] q.  A kernel of its own, apart from the chain's
+// (pass_up_lz): the pass is bound by VALU issue, and with the chain's scalars in
+// the same kernel the operator's launches spilled for them too (the 4x4 sector's
+// fp32 form 54 scalar registers and 24 bytes of scratch a lane, now 18 and none,
+// and 55 vector registers of 71: 0.517 -> 0.514 ms a launch; fp64 1.199 -> 1.190).
+template <typename T, int C, int RPT, int UKCH, bool LREG, bool COL, bool H16, bool SGN, int PFR = 0>
+static __device__ __forceinline__ void pass_up_op(const TwoPassView& V, const InterParams& I,
+                                                  const T* __restrict__ lut_up, const T* __restrict__ q,
+                                                  T* __restrict__ tout) {
+  typedef typename Vec<T, C>::type VT;
+  T* lut;
+  VT* P = up_lds<T, C, H16>(V, lut_up, lut);
+  const int npan = (V.dimdw + C - 1) / C;
+  if (!H16)
+    for (int k = threadIdx.x; k < 256; k += blockDim.x) lut[k] = lut_up[k];
+  if constexpr (PFR > 0) {
+    // the block's first panel is staged as usual; each later one is
+    // loaded into registers (PanelPrefetch) before the barrier that ends
+    // the current panel and written to P after it
+    const int dimup = V.dimup;
+    int pan = blockIdx.x;
+    if (pan >= npan) return;
+    stage_plain<T, C>(V, P, q, pan * C);
+    __syncthreads();
+    for (;;) {
+      const int nxt = pan + (int)gridDim.x;
+      up_rows<T, C, RPT, UKCH, LREG, COL, H16, SGN>(V, I, lut, P, tout, pan * C, (T)1);
+      if (nxt >= npan) break;
+      // the next panel's loads go out as soon as this thread's rows are
+      // done, so their round trip overlaps the other waves' last rows and
+      // the barrier (the waves of a block end an iteration apart)
+      PanelPrefetch<T, C, PFR> pf;
+      const int c1 = nxt * C;
 #pragma unroll
-        for (int j = 0; j < C; ++j)
-#pragma unroll
-          for (int kk = 0; kk < PFR; ++kk) {
-            const int r = (int)threadIdx.x + kk * (int)blockDim.x;
-            pf.v[j][kk] = (r < dimup && c1 + j < V.dimdw)
-                              ? __builtin_nontemporal_load(&qa[(size_t)(c1 + j) * V.ld + r])
-                              : (T)0;
-          }
-        __syncthreads();
+      for (int j = 0; j < C; ++j)
 #pragma unroll
         for (int kk = 0; kk < PFR; ++kk) {
           const int r = (int)threadIdx.x + kk * (int)blockDim.x;
-          if (r < dimup) {
-            VT x;
-#pragma unroll
-            for (int j = 0; j < C; ++j) Vec<T, C>::set(x, j, pf.v[j][kk]);
-            P[r] = x;
-          }
+          pf.v[j][kk] = (r < dimup && c1 + j < V.dimdw)
+                            ? __builtin_nontemporal_load(&q[(size_t)(c1 + j) * V.ld + r])
+                            : (T)0;
         }
-        __syncthreads();
-        pan = nxt;
+      __syncthreads();
+#pragma unroll
+      for (int kk = 0; kk < PFR; ++kk) {
+        const int r = (int)threadIdx.x + kk * (int)blockDim.x;
+        if (r < dimup) {
+          VT x;
+#pragma unroll
+          for (int j = 0; j < C; ++j) Vec<T, C>::set(x, j, pf.v[j][kk]);
+          P[r] = x;
+        }
       }
-      return;
+      __syncthreads();
+      pan = nxt;
     }
-    for (int pan = blockIdx.x; pan < npan; pan += gridDim.x)
-      up_panel<T, C, RPT, UKCH, LREG, COL, H16, SGN>(V, I, lut, P, qa, tout, pan * C, (T)1);
     return;
   }
+  for (int pan = blockIdx.x; pan < npan; pan += gridDim.x)
+    up_panel<T, C, RPT, UKCH, LREG, COL, H16, SGN>(V, I, lut, P, q, tout, pan * C, (T)1);
+}
+
+// A chain's step: phase B of the previous step where one is pending (r = t -
+// alpha_k v_k over t, block partial of |r|^2 into L.part_up, replay term
+// x += c_k v_k), then T = [D + H_up] q (unscaled; the down pass divides by s).
+// When the chain has run its nmax steps only the replay term remains.  TWO: steps
+// of two launches (L.sc2 set).
+template <typename T, int C, int RPT, int UKCH, bool LREG, bool COL, bool H16, bool SGN, bool TWO>
+static __device__ __forceinline__ void pass_up_lz(const TwoPassView& V, const InterParams& I,
+                                                  const T* __restrict__ lut_up, T* qa, T* qb,
+                                                  T* __restrict__ tout, const LzChain& L) {
+  typedef typename Vec<T, C>::type VT;
+  __shared__ double sh[16];
+  T* lut;
+  VT* P = up_lds<T, C, H16>(V, lut_up, lut);
+  const int npan = (V.dimdw + C - 1) / C;
   LzScalars s = *L.sc;
-  if (L.sc2) {
+  if constexpr (TWO) {
     // two-launch steps: alpha of the step before, the scalars to the down pass
+    // (member by member: a copied struct took 24 bytes of scratch a lane)
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (!s.stopped && s.pad == 3) {
       s.alpha_k = block_sum_of(L.part_dw, L.ndw, sh);
       s.nsteps = s.k + 1;
       s.pad = 1;
-      if (blockIdx.x == 0 && threadIdx.x == 0) L.alpha[s.k] = s.alpha_k;
+      if (lead) L.alpha[s.k] = s.alpha_k;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      LzScalars n = s;
-      if (s.pad && s.k + 1 >= L.nmax) n.stopped = 1;
-      *L.sc2 = n;
+    if (lead) {
+      LzScalars& n = *L.sc2;
+      n.k = s.k;
+      n.stopped = (s.stopped || (s.pad && s.k + 1 >= L.nmax)) ? 1 : 0;
+      n.nsteps = s.nsteps;
+      n.pad = s.pad;
+      n.s_cur = s.s_cur;
+      n.s_old = s.s_old;
+      n.beta_k = s.beta_k;
+      n.alpha_k = s.alpha_k;
+      n.norm2 = s.norm2;
     }
   }
   if (s.stopped) return;
@@ -497,28 +527,35 @@ static __device__ __forceinline__ void pass_up_body(const TwoPassView& V, const 
 }
 
 template <typename T, int C, int RPT, int UKCH, bool LREG = false, bool COL = false, bool H16 = false>
-__global__ __launch_bounds__(1024) void k_pass_up(TwoPassView V, InterParams I, const T* __restrict__ lut_up, T* qa,
-                                                  T* qb, T* __restrict__ tout, LzChain L, int chain) {
-  pass_up_body<T, C, RPT, UKCH, LREG, COL, H16, false>(V, I, lut_up, qa, qb, tout, L, chain);
+__global__ __launch_bounds__(1024) void k_pass_up(TwoPassView V, InterParams I, const T* __restrict__ lut_up,
+                                                  const T* __restrict__ q, T* __restrict__ tout) {
+  pass_up_op<T, C, RPT, UKCH, LREG, COL, H16, false>(V, I, lut_up, q, tout);
 }
 
 // The bank-scheduled two-hop passes (SGN: the words split by sign) with the
 // block's next panel loaded into registers as each thread finishes the
-// current one (operator mode; DimUp <= kUpPrefetchRows * blockDim; a chain
+// current one (operator only; DimUp <= kUpPrefetchRows * blockDim; a chain
 // step runs the form without it).
 template <typename T, int C, int RPT, int UKCH, bool SGN>
-__global__ __launch_bounds__(1024) void k_pass_upp(TwoPassView V, InterParams I, const T* __restrict__ lut_up, T* qa,
-                                                   T* qb, T* __restrict__ tout, LzChain L, int chain) {
-  pass_up_body<T, C, RPT, UKCH, true, true, true, SGN, kUpPrefetchRows>(V, I, lut_up, qa, qb, tout, L, chain);
+__global__ __launch_bounds__(1024) void k_pass_upp(TwoPassView V, InterParams I, const T* __restrict__ lut_up,
+                                                   const T* __restrict__ q, T* __restrict__ tout) {
+  pass_up_op<T, C, RPT, UKCH, true, true, true, SGN, kUpPrefetchRows>(V, I, lut_up, q, tout);
 }
 
 // The same pass reading the bank-scheduled two-hop words split by sign
 // (ColorTable::words16s): one coefficient per word for the whole wave, so a
 // hop costs no sign decoding.
 template <typename T, int C, int RPT, int UKCH>
-__global__ __launch_bounds__(1024) void k_pass_ups(TwoPassView V, InterParams I, const T* __restrict__ lut_up, T* qa,
-                                                   T* qb, T* __restrict__ tout, LzChain L, int chain) {
-  pass_up_body<T, C, RPT, UKCH, true, true, true, true>(V, I, lut_up, qa, qb, tout, L, chain);
+__global__ __launch_bounds__(1024) void k_pass_ups(TwoPassView V, InterParams I, const T* __restrict__ lut_up,
+                                                   const T* __restrict__ q, T* __restrict__ tout) {
+  pass_up_op<T, C, RPT, UKCH, true, true, true, true>(V, I, lut_up, q, tout);
+}
+
+// The chain forms of k_pass_up and k_pass_ups (SGN).
+template <typename T, int C, int RPT, int UKCH, bool LREG, bool COL, bool H16, bool SGN, bool TWO>
+__global__ __launch_bounds__(1024) void k_pass_up_lz(TwoPassView V, InterParams I, const T* __restrict__ lut_up, T* qa,
+                                                     T* qb, T* __restrict__ tout, LzChain L) {
+  pass_up_lz<T, C, RPT, UKCH, LREG, COL, H16, SGN, TWO>(V, I, lut_up, qa, qb, tout, L);
 }
 
 // ------------------------------------------------------------------ pass D
@@ -1572,14 +1609,27 @@ TwoPassView two_pass_view(const Sector& s, int ld) {
   return v;
 }
 
+template <typename T, int C, int RPT, int UKCH, bool LREG, bool COL, bool H16, bool SGN, bool TWO>
+static void launch_up_lz(const TwoPassView& V, const InterParams& I, const T* lut, T* qa, T* qb, T* tout,
+                         const LzChain& L, size_t lds, int grid, int threads, hipStream_t st) {
+  const auto f = k_pass_up_lz<T, C, RPT, UKCH, LREG, COL, H16, SGN, TWO>;
+  set_lds_limit((const void*)f, lds_limit_bytes() - 256);
+  hipLaunchKernelGGL(f, dim3(grid), dim3(threads), lds, st, V, I, lut, qa, qb, tout, L);
+  EDL_HIP(hipGetLastError());
+}
+
 template <typename T, int C, int RPT, int UKCH, bool LREG, bool COL, bool H16 = false>
 static void launch_up_l(const TwoPassView& V, const InterParams& I, const T* lut, T* qa, T* qb, T* tout,
                         const LzChain* L, int grid, int threads, hipStream_t st) {
   const size_t lds = H16 ? (size_t)(V.dimup + 32) * C * sizeof(T) : up_lds_bytes(V.dimup, C, sizeof(T));
   EDL_CHECK(lds <= (size_t)lds_limit_bytes() - 256, "launch_pass_up: panel exceeds LDS");
+  if (L && L->sc2)
+    return launch_up_lz<T, C, RPT, UKCH, LREG, COL, H16, false, true>(V, I, lut, qa, qb, tout, *L, lds, grid, threads, st);
+  if (L)
+    return launch_up_lz<T, C, RPT, UKCH, LREG, COL, H16, false, false>(V, I, lut, qa, qb, tout, *L, lds, grid, threads, st);
   set_lds_limit((const void*)k_pass_up<T, C, RPT, UKCH, LREG, COL, H16>, lds_limit_bytes() - 256);
   hipLaunchKernelGGL((k_pass_up<T, C, RPT, UKCH, LREG, COL, H16>), dim3(grid), dim3(threads), lds, st, V, I, lut, qa,
-                     qb, tout, L ? *L : LzChain{}, L ? 1 : 0);
+                     tout);
   EDL_HIP(hipGetLastError());
 }
 
@@ -1611,21 +1661,23 @@ static void launch_up_s(const TwoPassView& V, const InterParams& I, const T* lut
                         const LzChain* L, int grid, int threads, hipStream_t st) {
   const size_t lds = (size_t)(V.dimup + 32) * C * sizeof(T);
   EDL_CHECK(lds <= (size_t)lds_limit_bytes() - 256, "launch_pass_up: panel exceeds LDS");
+  if (L && L->sc2)
+    return launch_up_lz<T, C, RPT, UKCH, true, true, true, true, true>(V, I, lut, qa, qb, tout, *L, lds, grid, threads, st);
+  if (L)
+    return launch_up_lz<T, C, RPT, UKCH, true, true, true, true, false>(V, I, lut, qa, qb, tout, *L, lds, grid, threads, st);
   set_lds_limit((const void*)k_pass_ups<T, C, RPT, UKCH>, lds_limit_bytes() - 256);
-  hipLaunchKernelGGL((k_pass_ups<T, C, RPT, UKCH>), dim3(grid), dim3(threads), lds, st, V, I, lut, qa, qb, tout,
-                     L ? *L : LzChain{}, L ? 1 : 0);
+  hipLaunchKernelGGL((k_pass_ups<T, C, RPT, UKCH>), dim3(grid), dim3(threads), lds, st, V, I, lut, qa, tout);
   EDL_HIP(hipGetLastError());
 }
 
 template <typename T, int C, int RPT, int UKCH, bool SGN>
-static void launch_up_p(const TwoPassView& V, const InterParams& I, const T* lut, T* qa, T* qb, T* tout,
-                        const LzChain* L, int grid, int threads, hipStream_t st) {
+static void launch_up_p(const TwoPassView& V, const InterParams& I, const T* lut, const T* q, T* tout, int grid,
+                        int threads, hipStream_t st) {
   const size_t lds = (size_t)(V.dimup + 32) * C * sizeof(T);
   EDL_CHECK(lds <= (size_t)lds_limit_bytes() - 256, "launch_pass_up: panel exceeds LDS");
   EDL_CHECK(V.dimup <= kUpPrefetchRows * threads, "launch_pass_up: the prefetching form takes DimUp <= kUpPrefetchRows * threads");
   set_lds_limit((const void*)k_pass_upp<T, C, RPT, UKCH, SGN>, lds_limit_bytes() - 256);
-  hipLaunchKernelGGL((k_pass_upp<T, C, RPT, UKCH, SGN>), dim3(grid), dim3(threads), lds, st, V, I, lut, qa, qb, tout,
-                     L ? *L : LzChain{}, L ? 1 : 0);
+  hipLaunchKernelGGL((k_pass_upp<T, C, RPT, UKCH, SGN>), dim3(grid), dim3(threads), lds, st, V, I, lut, q, tout);
   EDL_HIP(hipGetLastError());
 }
 
@@ -1634,9 +1686,11 @@ static void launch_up_k(const TwoPassView& V, const InterParams& I, const T* lut
                         const LzChain* L, int grid, int threads, int col, hipStream_t st) {
   if (col == 5 || col == 6) {
     EDL_CHECK(up_col_ok(V, C, sizeof(T), col), "launch_pass_up: no two-hop bank-scheduled table for this form");
+    // (a chain step runs the form without the prefetch)
+    if (L) return launch_up_k<T, C, RPT, UKCH>(V, I, lut, qa, qb, tout, L, grid, threads, col == 5 ? 2 : 4, st);
     if constexpr ((sizeof(T) == 8 && C == 1) || (sizeof(T) == 4 && (C == 1 || C == 3))) {
-      if (col == 5) return launch_up_p<T, C, RPT, UKCH, false>(V, I, lut, qa, qb, tout, L, grid, threads, st);
-      return launch_up_p<T, C, RPT, UKCH, true>(V, I, lut, qa, qb, tout, L, grid, threads, st);
+      if (col == 5) return launch_up_p<T, C, RPT, UKCH, false>(V, I, lut, qa, tout, grid, threads, st);
+      return launch_up_p<T, C, RPT, UKCH, true>(V, I, lut, qa, tout, grid, threads, st);
     }
   }
   if (col == 4) {
