@@ -2284,7 +2284,7 @@ static BtShape bt_tune(Ctx& c, const std::vector<BtChain>& chains, int max_up, i
     BtSet bs;
     bs.shape = shp;
     bs.h = bt_resized(chains, shp);
-    bt_finalize<T>(bs);
+    bt_finalize<T>(bs, st);
     for (int r = 0; r < 3; ++r) {
       if (r == 1) EDL_HIP(hipStreamSynchronize(st));
       EventTimer tm(st);
@@ -2398,7 +2398,7 @@ static bool bt_pick_persist(Ctx& c, const std::vector<BtChain>& chains, const Bt
       bs.shape = shp;
       bs.h = bt_resized(chains, shp);
       for (BtChain& b : bs.h) b.nmax = 1;
-      bt_finalize<T>(bs);
+      bt_finalize<T>(bs, st);
       double best = 1e300;
       for (int r = 0; r < 2; ++r) {
         restore();
@@ -2692,14 +2692,14 @@ static int64_t tridiag_group(Ctx& c, const std::vector<SeedSpec>& seeds, const s
     if (nstreams == 1) {
       bs.shape = shp;
       bs.h = bt_resized(btchains, shp);
-      bt_finalize<T>(bs);
+      bt_finalize<T>(bs, st);
     } else {
       const std::vector<BtChain> all = bt_resized(btchains, shp);
       parts.resize(nstreams);
       for (int h = 0; h < nstreams; ++h) {
         parts[h].shape = shp;
         parts[h].h.assign(all.begin() + all.size() * h / nstreams, all.begin() + all.size() * (h + 1) / nstreams);
-        bt_finalize<T>(parts[h]);
+        bt_finalize<T>(parts[h], st);
       }
     }
   }

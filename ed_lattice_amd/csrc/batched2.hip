@@ -610,7 +610,7 @@ static void bt_attributes() {
 }
 
 template <typename T>
-void bt_finalize(BtSet& bs) {
+void bt_finalize(BtSet& bs, hipStream_t st) {
   bt_attributes<T>();
   const size_t n = bs.h.size();
   std::vector<int64_t> tu(n + 1, 0), td(n + 1, 0);
@@ -622,21 +622,23 @@ void bt_finalize(BtSet& bs) {
   }
   bs.tiles_up = tu[n];
   bs.tiles_dw = td[n];
-  bs.d = static_cast<BtChain*>(dev_alloc(sizeof(BtChain) * n));
-  bs.d_tile_up = static_cast<int64_t*>(dev_alloc(sizeof(int64_t) * (n + 1)));
-  bs.d_tile_dw = static_cast<int64_t*>(dev_alloc(sizeof(int64_t) * (n + 1)));
-  EDL_HIP(hipMemcpy(bs.d, bs.h.data(), sizeof(BtChain) * n, hipMemcpyHostToDevice));
-  EDL_HIP(hipMemcpy(bs.d_tile_up, tu.data(), sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice));
-  EDL_HIP(hipMemcpy(bs.d_tile_dw, td.data(), sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice));
   std::vector<int32_t> cu((size_t)bs.tiles_up), cdw((size_t)bs.tiles_dw);
   for (size_t k = 0; k < n; ++k) {
     for (int64_t t = tu[k]; t < tu[k + 1]; ++t) cu[(size_t)t] = (int32_t)k;
     for (int64_t t = td[k]; t < td[k + 1]; ++t) cdw[(size_t)t] = (int32_t)k;
   }
-  bs.d_chain_up = static_cast<int32_t*>(dev_alloc(sizeof(int32_t) * std::max<size_t>(cu.size(), 1)));
-  bs.d_chain_dw = static_cast<int32_t*>(dev_alloc(sizeof(int32_t) * std::max<size_t>(cdw.size(), 1)));
-  EDL_HIP(hipMemcpy(bs.d_chain_up, cu.data(), sizeof(int32_t) * cu.size(), hipMemcpyHostToDevice));
-  EDL_HIP(hipMemcpy(bs.d_chain_dw, cdw.data(), sizeof(int32_t) * cdw.size(), hipMemcpyHostToDevice));
+  auto up = [st](auto*& p, const auto& v) {
+    void* q = nullptr;
+    const hipError_t e = dev_upload(&q, v.data(), sizeof(v[0]) * v.size(), st);
+    p = static_cast<std::remove_reference_t<decltype(p)>>(q);  // (freed by ~BtSet, errors included)
+    EDL_HIP(e);
+  };
+  up(bs.d, bs.h);
+  up(bs.d_tile_up, tu);
+  up(bs.d_tile_dw, td);
+  up(bs.d_chain_up, cu);
+  up(bs.d_chain_dw, cdw);
+  EDL_HIP(hipStreamSynchronize(st));  // the host vectors must outlive the copies
 }
 
 bool bt_h16_ok(const std::vector<BtChain>& chains, int spin) {
@@ -787,8 +789,8 @@ void bt_launch_persist(const BtSet& bs, const InterParams& I, hipStream_t st) {
 
 template void bt_launch_persist<double>(const BtSet&, const InterParams&, hipStream_t);
 template void bt_launch_persist<float>(const BtSet&, const InterParams&, hipStream_t);
-template void bt_finalize<double>(BtSet&);
-template void bt_finalize<float>(BtSet&);
+template void bt_finalize<double>(BtSet&, hipStream_t);
+template void bt_finalize<float>(BtSet&, hipStream_t);
 template void bt_launch_up<double>(const BtSet&, const InterParams&, hipStream_t, bool);
 template void bt_launch_up<float>(const BtSet&, const InterParams&, hipStream_t, bool);
 template void bt_launch_dw<double>(const BtSet&, hipStream_t, bool);

@@ -76,7 +76,7 @@ struct BtSet {
 bool bt_h16_ok(const std::vector<BtChain>& chains, int spin);
 
 template <typename T>
-void bt_finalize(BtSet& bs);
+void bt_finalize(BtSet& bs, hipStream_t st);
 // One pass over every tile, then (scalars = true) the per-chain scalar
 // update that completes the step's half (beta after the up pass, alpha after
 // the down pass).  scalars = false launches the tile kernel alone and leaves

@@ -141,11 +141,12 @@ inline TwoPassCfg chain_cfg(const TwoPassCfg& c) {
   return r;
 }
 
-// Whether a chain with this schedule runs steps of two launches: the
-// vector-gather down pass, and few enough blocks that each can add up the other
+// Whether a chain with this schedule can run steps of two launches (the
+// vector-gather down pass), and whether it does: few enough blocks that each can add up the other
 // pass's partials.  Below the limit the two small launches cost more than the
 // sums (3x4, 853 776 states, 464 + 512 blocks); a block of the 4x4 sector's
 // 20 000 and more would spend its time on them.
+bool chain_fusable(const TwoPassCfg& cfg);
 bool chain_fused(const TwoPassView& V, const TwoPassCfg& cfg);
 
 // Whether the bank-scheduled up-pass table exists for panels of C columns of

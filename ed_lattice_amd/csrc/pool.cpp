@@ -146,6 +146,11 @@ void* dev_try_alloc(size_t bytes) {
   }
   return p;
 }
+hipError_t dev_upload(void** p, const void* src, size_t bytes, hipStream_t st) {
+  *p = dev_try_alloc(bytes);
+  if (!*p) return hipErrorOutOfMemory;
+  return bytes ? hipMemcpyAsync(*p, src, bytes, hipMemcpyHostToDevice, st) : hipSuccess;
+}
 void dev_free(void* p) {
   if (!p) return;
   if (DevPool* pool = current_pool())

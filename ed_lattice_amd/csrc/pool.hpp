@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <exception>
 #include <map>
 #include <mutex>
 
@@ -30,8 +31,10 @@ size_t device_cached_bytes();
 // when the context is destroyed, takes a model of another number of sites, or
 // an allocation of this library on the device fails (device_malloc, from any
 // context and thread).  All work of a context is ordered on
-// its stream, so a buffer put back while launches that use it are queued is
-// safe to hand to later launches.
+// its stream, copies into its buffers too (dev_upload), so a buffer put back
+// while launches that use it are queued is safe to hand to later launches; a
+// call's other streams are joined before their buffers go back, and a call that
+// ends with an exception waits for the device (PoolScope).
 class DevPool {
  public:
   DevPool();
@@ -56,12 +59,22 @@ class DevPool {
 DevPool*& current_pool();
 struct PoolScope {
   DevPool* before;
+  int unwinding = std::uncaught_exceptions();
   explicit PoolScope(DevPool& p) : before(current_pool()) { current_pool() = &p; }
-  ~PoolScope() { current_pool() = before; }
+  ~PoolScope() {
+    // the buffers of the call are back in the pool, with launches on any of its
+    // streams still queued: none may be handed out before those have run
+    if (std::uncaught_exceptions() > unwinding) (void)hipDeviceSynchronize();
+    current_pool() = before;
+  }
   PoolScope(const PoolScope&) = delete;
   PoolScope& operator=(const PoolScope&) = delete;
 };
 void* dev_try_alloc(size_t bytes);  // nullptr (no error left pending) when there is no memory
 void dev_free(void* p);
+// dev_try_alloc and a copy of host memory into it, on the stream: the copy comes
+// after the launches queued there that a kept buffer may still serve.  `src` has
+// to live until the stream is waited for.
+hipError_t dev_upload(void** p, const void* src, size_t bytes, hipStream_t st);
 
 }  // namespace edl

@@ -14,13 +14,19 @@ RUNTIME = r"""
 #include <cstdint>
 #include <map>
 #include <mutex>
+#include <utility>
+#include <vector>
 typedef int hipError_t;
+typedef void* hipStream_t;
 enum { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2 };
 struct Sim {
   std::recursive_mutex m;
   size_t total = (size_t)16 << 20, used[2] = {0, 0};
   std::map<void*, std::pair<int, size_t>> at;
   int pending = 0, syncs = 0;
+  // launches and copies queued and not waited for: stream, buffer
+  std::vector<std::pair<void*, void*>> queued;
+  std::vector<void*> late;  // buffers written while another stream still used them
 };
 inline Sim& sim() { static Sim s; return s; }
 inline int& sim_device() { static thread_local int d = 0; return d; }
@@ -50,7 +56,15 @@ inline hipError_t hipMemGetInfo(size_t* f, size_t* t) {
   *f = sim().total - sim().used[sim_device()];
   return hipSuccess;
 }
-inline hipError_t hipDeviceSynchronize() { ++sim().syncs; return hipSuccess; }
+inline hipError_t hipDeviceSynchronize() { ++sim().syncs; sim().queued.clear(); return hipSuccess; }
+inline void sim_use(void* st, void* p) {
+  for (auto& q : sim().queued)
+    if (q.second == p && q.first != st) sim().late.push_back(p);
+  sim().queued.push_back({st, p});
+}
+enum { hipMemcpyHostToDevice = 1 };
+inline hipError_t hipMemcpyAsync(void* d, const void*, size_t, int, hipStream_t st) { sim_use(st, d); return hipSuccess; }
+inline hipError_t hipMemcpy(void* d, const void*, size_t, int) { sim_use(nullptr, d); return hipSuccess; }
 """
 
 HEAD = r"""
@@ -121,6 +135,43 @@ CASES = {
   (void)hipGetLastError();
   WANT(a.cached() == 0 && b.cached() >= 900 * K);
 """,
+    # a buffer put back with launches queued and filled again: on the same stream
+    "upload": r"""
+  DevPool a;
+  PoolScope s(a);
+  int main_stream = 0;
+  const char host[64] = {};
+  void* x = dev_try_alloc(64);
+  sim_use(&main_stream, x);
+  dev_free(x);
+  void* y = nullptr;
+  WANT(dev_upload(&y, host, 64, &main_stream) == hipSuccess && y == x && sim().late.empty());
+  dev_free(y);
+  WANT(sim().syncs == 0);
+""",
+    # a call that ends with an exception and launches queued on a second stream
+    "unwind": r"""
+  DevPool a;
+  int main_stream = 0, second = 0;
+  void* used = nullptr;
+  try {
+    PoolScope s(a);
+    struct Buf { void* p = dev_try_alloc(64); ~Buf() { dev_free(p); } } b;
+    used = b.p;
+    sim_use(&second, b.p);
+    throw std::runtime_error("launch failed");
+  } catch (const std::exception&) {
+  }
+  WANT(current_pool() == nullptr && sim().syncs == 1);
+  {
+    PoolScope s(a);
+    void* x = dev_try_alloc(64);
+    WANT(x == used);
+    sim_use(&main_stream, x);
+    dev_free(x);
+  }
+  WANT(sim().late.empty() && sim().syncs == 1);  // a call that ends well does not wait
+""",
     # two contexts on threads of their own, both short of memory
     "threads": r"""
   DevPool a, b;
@@ -155,6 +206,12 @@ def test_pool(case, tmp_path):
                     os.path.join(CSRC, "pool.cpp")], check=True)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
+
+
+def test_buffers_filled_on_the_stream():
+    """No kept buffer of the batched chains is filled outside the context's stream."""
+    with open(os.path.join(CSRC, "batched2.hip")) as f:
+        assert "hipMemcpy(" not in f.read()
 
 
 def test_every_allocation_can_take_the_cache_back():
