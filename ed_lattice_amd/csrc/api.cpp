@@ -18,6 +18,7 @@
 #include "resident.hpp"
 #include "seeds.hpp"
 #include "tridiag.hpp"
+#include "tune_time.hpp"
 
 struct edl_ctx {
   edl::Ctx c;
@@ -297,10 +298,52 @@ static bool two_pass_pin(const TwoPassView& V, TwoPassCfg& best) {
   return false;
 }
 
+// The events of a tuning run.
+struct TuneClock {
+  hipEvent_t a = nullptr, b = nullptr;
+  hipStream_t st;
+  explicit TuneClock(hipStream_t s) : st(s) {
+    EDL_HIP(hipEventCreate(&a));
+    if (hipEventCreate(&b) != hipSuccess) {
+      (void)hipEventDestroy(a);
+      throw Error("hipEventCreate failed");
+    }
+  }
+  TuneClock(const TuneClock&) = delete;
+  TuneClock& operator=(const TuneClock&) = delete;
+  ~TuneClock() {
+    (void)hipEventDestroy(a);
+    (void)hipEventDestroy(b);
+  }
+  // ms of n launches queued one after another.
+  template <typename Launch>
+  double run(Launch launch, int n) {
+    EDL_HIP(hipEventRecord(a, st));
+    for (int r = 0; r < n; ++r) launch();
+    EDL_HIP(hipEventRecord(b, st));
+    EDL_HIP(hipEventSynchronize(b));
+    float t = 0.f;
+    EDL_HIP(hipEventElapsedTime(&t, a, b));
+    return t;
+  }
+  // Mean ms of a launch, or of the one that shows it to be slower than the best
+  // (candidate_ms).
+  template <typename Launch>
+  double ms(Launch launch, double best_ms) {
+    return candidate_ms(launch, [&](int n) { return run(launch, n); }, best_ms);
+  }
+  // ms of a warm call that is waited for, the least of twelve.
+  template <typename Launch>
+  double alone(Launch launch) {
+    launch();
+    double t = 1e300;
+    for (int r = 0; r < 12; ++r) t = std::min(t, run(launch, 1));
+    return t;
+  }
+};
+
 // Pick panel widths, block sizes and grids of the two passes by timing the
-// operator on the sector itself, in the layout it will run on (ld): a first
-// launch of each candidate, and three more where that one was not slower
-// than twice the best so far.
+// operator on the sector itself, in the layout it will run on (ld).
 template <typename T>
 static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s, int ld) {
   const TwoPassView V = two_pass_view(s, ld);
@@ -322,16 +365,8 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s, int ld) {
     EDL_HIP(hipStreamSynchronize(st));
   }
   const int lds = 160 * 1024;
-  // mean ms of one launch
-  auto timed = [&](const std::function<void()>& launch, double best_ms) {
-    EventTimer first(st);
-    launch();
-    const double one = first.stop();
-    if (one > 2.0 * best_ms) return one;
-    EventTimer tm(st);
-    for (int r = 0; r < 3; ++r) launch();
-    return tm.stop() / 3;
-  };
+  TuneClock clock(st);
+  auto timed = [&](const std::function<void()>& launch, double best_ms) { return clock.ms(launch, best_ms); };
   {
     best.grid_up = c.num_cu;
     best.nchunk = std::min(32, V.dimdw);
@@ -432,25 +467,37 @@ static TwoPassCfg two_pass_cfg(Ctx& c, const Sector& s, int ld) {
           }
         }
   }
-  // the one-launch form against the two passes together
+  // The one-launch form against the two passes together, as a caller has them, each
+  // call waited for: the least of twelve such repeats within 0.2 us, where means of
+  // three in a row (which hide the second launch) or of fewer single ones took the
+  // two passes or another shape now and then, on sectors of 2 000 to 140 000 states
+  // 18.6 to 23.3 us a call for 17.4 to 18.1.
   if (one_pass_size(s, sizeof(T))) {
     auto two = [&]() {
       launch_pass_up<T>(V, c.model.inter, lut_dev<T>(s.sp[0]), q.as<T>(), q.as<T>(), t.as<T>(), nullptr, best, st);
       launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), q.as<T>(), q.as<T>(), t.as<T>(), o.as<T>(), nullptr, best, st);
     };
-    double best_ms = one_pass_pin() == 1 ? 1e300 : std::min(timed(two, 1e300), timed(two, 1e300));
-    for (const TwoPassCfg& w : one_pass_shapes(V, best, sizeof(T))) {
-      const double ms = timed([&]() {
+    TwoPassCfg one = best;
+    auto cols = [&](const TwoPassCfg& w) {
+      return [&, w]() {
         launch_cols<T>(V, c.model.inter, lut_dev<T>(s.sp[0]), lut_dev<T>(s.sp[1]), q.as<T>(), o.as<T>(), w, st);
-      }, best_ms);
+      };
+    };
+    double best_ms = 1e300;
+    for (const TwoPassCfg& w : one_pass_shapes(V, best, sizeof(T))) {
+      const double ms = clock.alone(cols(w));
       if (verbose())
-        std::fprintf(stderr, "[edl] tune one launch fp%d C %d threads %4d (best so far %.4f): %.4f ms\n",
-                     8 * (int)sizeof(T), w.one_C, w.one_threads, best_ms, ms);
+        std::fprintf(stderr, "[edl] tune one launch fp%d C %d threads %4d: %.4f ms\n", 8 * (int)sizeof(T), w.one_C,
+                     w.one_threads, ms);
       if (ms < best_ms) {
         best_ms = ms;
-        best.one_C = w.one_C;
-        best.one_threads = w.one_threads;
+        one = w;
       }
+    }
+    if (one.one_C > 0) {
+      const double a1 = clock.alone(cols(one)), a2 = clock.alone(two);
+      if (verbose()) std::fprintf(stderr, "[edl] tune alone: one launch %.4f ms, two passes %.4f ms\n", a1, a2);
+      if (one_pass_pin() == 1 || a1 < a2) best = one;
     }
   }
   tp_cache()[key] = best;
@@ -488,6 +535,7 @@ static TwoPassCfg two_pass_chain_cfg(Ctx& c, const Sector& s) {
     return best;
   }
   hipStream_t st = c.stream;
+  TuneClock clock(st);
   const int64_t D = s.dim, Dp = (int64_t)ld * s.sp[1].dim;
   DevBuf d64(sizeof(double) * D), q(sizeof(T) * Dp), t(sizeof(T) * Dp), o(sizeof(T) * Dp);
   launch_start_vector(d64.as<double>(), D, 0x5EEDull, st);
@@ -546,14 +594,12 @@ static TwoPassCfg two_pass_chain_cfg(Ctx& c, const Sector& s) {
             w.dw_rng = 0;
             w.dw_ord = ord;
             if (pass_dw_lds_bytes(V, w) > (size_t)lds - 4096) continue;
-            launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), q.as<T>(), o.as<T>(), t.as<T>(), nullptr, &A, w, st);
-            EventTimer tm(st);
-            for (int r = 0; r < 3; ++r)
+            const double ms = clock.ms([&]() {
               launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), q.as<T>(), o.as<T>(), t.as<T>(), nullptr, &A, w, st);
-            const double ms = tm.stop();
+            }, bc);
             if (verbose())
               std::fprintf(stderr, "[edl] tune dw chain fp%d ord %d R %3d ncol %d kch %d threads %4d chunks %3d: %.4f ms\n",
-                           8 * (int)sizeof(T), ord, R, w.ncol, w.kch, th, nch, ms / 3);
+                           8 * (int)sizeof(T), ord, R, w.ncol, w.kch, th, nch, ms);
             if (ms < bc) {
               bc = ms;
               best.ch_R = R;
@@ -575,14 +621,12 @@ static TwoPassCfg two_pass_chain_cfg(Ctx& c, const Sector& s) {
           w.threads_dw = th;
           w.dw_rng = b;
           w.dw_vec = 0;
-          launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), q.as<T>(), o.as<T>(), t.as<T>(), nullptr, &A, w, st);
-          EventTimer tm(st);
-          for (int r = 0; r < 3; ++r)
+          const double ms = clock.ms([&]() {
             launch_pass_dw<T>(V, lut_dev<T>(s.sp[1]), q.as<T>(), o.as<T>(), t.as<T>(), nullptr, &A, w, st);
-          const double ms = tm.stop();
+          }, bc);
           if (verbose())
             std::fprintf(stderr, "[edl] tune dw chain fp%d ranges b %d R %3d threads %4d: %.4f ms\n",
-                         8 * (int)sizeof(T), b, R, th, ms / 3);
+                         8 * (int)sizeof(T), b, R, th, ms);
           if (ms < bc) {
             bc = ms;
             best.ch_R = R;
@@ -616,14 +660,12 @@ static TwoPassCfg two_pass_chain_cfg(Ctx& c, const Sector& s) {
             w.threads_up = th;
             w.grid_up = c.num_cu * gm;
             // qa = q_k (q), qb = t (o): phase B reads both and rewrites t
-            launch_pass_up<T>(V, c.model.inter, lut_dev<T>(s.sp[0]), q.as<T>(), o.as<T>(), t.as<T>(), &A, w, st);
-            EventTimer tm(st);
-            for (int r = 0; r < 3; ++r)
+            const double ms = clock.ms([&]() {
               launch_pass_up<T>(V, c.model.inter, lut_dev<T>(s.sp[0]), q.as<T>(), o.as<T>(), t.as<T>(), &A, w, st);
-            const double ms = tm.stop();
+            }, bu2);
             if (verbose())
               std::fprintf(stderr, "[edl] tune up chain fp%d C %d col %d rpt %d kch %2d threads %4d grid %5d: %.4f ms\n",
-                           8 * (int)sizeof(T), C, col, w.up_rpt, w.up_kch, th, w.grid_up, ms / 3);
+                           8 * (int)sizeof(T), C, col, w.up_rpt, w.up_kch, th, w.grid_up, ms);
             if (ms < bu2) {
               bu2 = ms;
               best.ch_C = C;
@@ -1015,8 +1057,7 @@ static Schedule autotune(Ctx& c, const std::vector<ChainDev>& chains, hipStream_
   return best;
 }
 
-// Run the chain set until every chain has stopped or `steps` steps, with the
-// two phases of a step captured once in a hipGraph and replayed.  With
+// Run the chain set until every chain has stopped or `steps` steps.  With
 // check > 0 and a single chain, the lowest Ritz value is checked every
 // `check` steps and the run ends when it changes by <= tol*|E|.
 // Phase A of a single large chain done by the two-pass operator.
