@@ -1077,6 +1077,13 @@ struct TwoPassStep {
   double* defl_coef = nullptr;
 };
 
+// EDL_TWO_LAUNCH=0|1 keeps the steps of single chains off the two-launch form, or
+// takes it at any number of blocks (and fails where a chain has no such form).
+static int two_launch_pin() {
+  const char* e = std::getenv("EDL_TWO_LAUNCH");
+  return e && *e ? std::atoi(e) : -1;
+}
+
 // The buffers a chain's steps share: the two-pass intermediate, the partial
 // sums and, for two-launch steps, the second place of the scalars (after
 // part_dw).
@@ -1090,7 +1097,13 @@ static void chain_buffers(Ctx& c, TwoPassStep<T>& tps, bool seg, bool deflate, c
   dw = DevBuf(sizeof(double) * ndw + sizeof(LzScalars));
   tps.L.part_up = up.as<double>();
   tps.L.part_dw = dw.as<double>();
-  if (!phase_b && !S.nonlocal && chain_fused(tps.V, tps.cfg)) {
+  const int pin = two_launch_pin();
+  const bool can = !phase_b && !S.nonlocal && chain_fusable(tps.cfg);
+  EDL_CHECK(pin != 1 || can, "EDL_TWO_LAUNCH=1: this chain's steps cannot run in two launches");
+  const bool two = can && pin != 0 && (pin == 1 || chain_fused(tps.V, tps.cfg));
+  if (verbose()) std::fprintf(stderr, "[edl] chain steps: %s\n", two ? "two launches" : "more than two launches");
+  if (verbose()) std::fprintf(stderr, "[edl] chain blocks: up %d, down %d\n", nup, ndw);
+  if (two) {
     tps.L.sc2 = reinterpret_cast<LzScalars*>(tps.L.part_dw + ndw);
     tps.L.nup = nup;
     tps.L.ndw = ndw;

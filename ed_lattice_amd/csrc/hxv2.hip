@@ -1796,9 +1796,10 @@ int pass_dw_grid(const TwoPassView& V, const TwoPassCfg& cfg) {
   return 8 * cfg.nchunk * ((npan + 7) / 8);
 }
 
-constexpr int kFusedBlocks = 2048;
+constexpr int kFusedBlocks = 6400;
+bool chain_fusable(const TwoPassCfg& cfg) { return cfg.dw_vec == 1 && cfg.dw_rng == 0; }
 bool chain_fused(const TwoPassView& V, const TwoPassCfg& cfg) {
-  return cfg.dw_vec == 1 && cfg.dw_rng == 0 && pass_dw_grid(V, cfg) <= kFusedBlocks;
+  return chain_fusable(cfg) && pass_dw_grid(V, cfg) <= kFusedBlocks;
 }
 
 static size_t pass_dwr_lds(const TwoPassView& V, int R, int b, size_t elem) {

@@ -142,10 +142,13 @@ inline TwoPassCfg chain_cfg(const TwoPassCfg& c) {
 }
 
 // Whether a chain with this schedule can run steps of two launches (the
-// vector-gather down pass), and whether it does: few enough blocks that each can add up the other
-// pass's partials.  Below the limit the two small launches cost more than the
-// sums (3x4, 853 776 states, 464 + 512 blocks); a block of the 4x4 sector's
-// 20 000 and more would spend its time on them.
+// vector-gather down pass), and whether it does: few enough blocks that each can
+// add up the other pass's partials for less than the two small launches cost.  us a
+// step, two launches and four, by the down pass's blocks: 464 29.7, 33.6 (3x4 fp32);
+// 1 512 72.5, 76.5 (13-ring (6,6) fp64); 3 456 152.4, 156.1 (2x7 (7,7) fp32); 6 280
+// 580, 587 (3x5 (6,6) fp64); 6 912 151.2, 150.1 (14-ring (7,7) fp32); 10 240 325, 319;
+// 11 584 242, 234 (14-ring (7,7) fp64); level again, or better, where a step takes 0.5
+// ms and more (3x5 (8,7) fp64, 20 560: 998, 1 050), which no rule on blocks tells apart.
 bool chain_fusable(const TwoPassCfg& cfg);
 bool chain_fused(const TwoPassView& V, const TwoPassCfg& cfg);
 
