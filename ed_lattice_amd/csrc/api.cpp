@@ -1353,11 +1353,39 @@ struct GsRun {
   int64_t hxv = 0;
 };
 
-// Small sectors (res_ok) run their chains resident, a chain to a block, unless
-// a pinned schedule or a forced segmentation asks for the two-pass step.
-static bool resident_sector(const Sector& S, size_t elem) {
-  return !std::getenv("EDL_UP_SEGMENT_ROWS") && !std::getenv("EDL_TWO_PASS_CFG_F32") &&
-         !std::getenv("EDL_TWO_PASS_CFG_F64") && res_ok(S, elem);
+static bool res_one(const Sector& S) { return S.sp[0].nvals <= 1 && S.sp[1].nvals <= 1; }
+
+// Elements a thread (of 1024) up to which a chain runs resident, a chain to a
+// block.  Beyond 8 in fp64 and 11 or so in fp32 an element's registers spill
+// (resident.hip), and the chip is filled only by as many chains as CUs; the other
+// forms take about the same time at all these sizes.  `chains` 0: a ground state,
+// against two-launch steps (120 steps, ms, resident and two-launch: fp64, one
+// hopping value, 7 056 states 1.88, 2.36; 9 075: 2.12, 2.24; 10 584: 2.70, 2.34;
+// 15 876: 4.60, 2.40; several values, 7 056: 2.12, 2.37; 8 281: 2.72, 2.25; fp32,
+// one, 11 340: 1.99, 2.35; 14 014: 2.66, 2.52; several, 9 504: 2.32, 2.47; 10 584:
+// 2.74, 2.37).  Otherwise a group of so many seeds, against the tiles (40 steps of
+// fp64 chains, one value, 14 520 states: 1 chain 1.19, 0.80; 32: 1.22, 1.20; 128:
+// 1.92, 2.74; several, 11 340: 1 chain 0.99, 0.79; 32: 1.01, 1.06; fp32, one, 15 876:
+// 1 chain 0.86, 0.79; 32: 0.90, 1.05; several, 11 340: 1 chain 0.85, 0.80; 14 520:
+// 1 chain 1.05, 0.80; 32: 1.09, 1.14).
+static int res_rows(size_t elem, bool one, size_t chains) {
+  const int at = chains == 0 ? 0 : (chains < 32 ? 1 : (chains < 128 ? 2 : 3));
+  static const int rows[2][2][4] = {{{8, 10, 12, 16}, {9, 12, 12, 16}},    // fp64: several values, one
+                                    {{9, 11, 16, 16}, {12, 14, 16, 16}}};  // fp32
+  return rows[elem == 4][one][at];
+}
+
+// Whether the chains of a group on S run resident: within res_rows, unless a
+// pinned schedule or a forced segmentation asks for the two-pass step.
+// EDL_RESIDENT=0|1 keeps chains off the form, or takes it wherever it fits
+// (res_ok).
+static bool resident_sector(const Sector& S, size_t elem, size_t chains) {
+  const char* e = std::getenv("EDL_RESIDENT");
+  const int pin = e && *e ? std::atoi(e) : -1;
+  if (pin == 0 || std::getenv("EDL_UP_SEGMENT_ROWS") || std::getenv("EDL_TWO_PASS_CFG_F32") ||
+      std::getenv("EDL_TWO_PASS_CFG_F64") || !res_ok(S, elem))
+    return false;
+  return pin == 1 || S.dim <= (int64_t)1024 * res_rows(elem, res_one(S), chains);
 }
 
 // The chain of a resident launch on sector S without its start and outputs.
@@ -1371,8 +1399,6 @@ static ResChain res_chain(const Sector& S, int nmax) {
   r.brk_tol = 1e-14;
   return r;
 }
-static bool res_one(const Sector& S) { return S.sp[0].nvals <= 1 && S.sp[1].nvals <= 1; }
-
 // Scalars and coefficients of one chain as a resident launch leaves them:
 // {LzScalars, alpha[nmax], beta[nmax]}, one device-to-host copy.
 static size_t res_out_bytes(int nmax) { return sizeof(LzScalars) + 2 * sizeof(double) * (size_t)nmax; }
@@ -1394,6 +1420,7 @@ static ChainOut res_out(const char* p, int nmax) {
 // adds up the eigenvector instead.
 template <typename T>
 static GsRun gs_run_resident(Ctx& c, Sector& S, const double* d_start, int nmax, double tol, int check, double* d_x) {
+  if (verbose()) std::fprintf(stderr, "[edl] chain steps: resident\n");
   hipStream_t st = c.stream;
   const int64_t D = S.dim;
   const size_t vbytes = sizeof(T) * (size_t)D;
@@ -1484,7 +1511,7 @@ static GsRun gs_run(Ctx& c, Sector& S, const double* d_start, int niter, double 
                     const double* d_X = nullptr, int nX = 0) {
   hipStream_t st = c.stream;
   const int nmax = (int)std::min<int64_t>(niter, S.dim);
-  if (nX == 0 && resident_sector(S, sizeof(T)))
+  if (nX == 0 && resident_sector(S, sizeof(T), 0))
     return gs_run_resident<T>(c, S, d_start, nmax, tol, check, d_x);
   GsRun r;
   Schedule sch;
@@ -2507,6 +2534,7 @@ static int64_t tridiag_resident(Ctx& c, const std::vector<SeedSpec>& seeds, cons
   hipStream_t st = c.stream;
   const size_t n = idx.size();
   if (n == 0) return 0;
+  if (verbose()) std::fprintf(stderr, "[edl] chain steps: resident\n");
   std::vector<ResChain> r(n);
   std::vector<size_t> at(n + 1, 0);
   int64_t max_dim = 1;
@@ -2577,7 +2605,8 @@ static int64_t tridiag_group(Ctx& c, const std::vector<SeedSpec>& seeds, const s
     // small targets: resident chains, unless EDL_BATCHED_KERNELS forces a form
     const char* e = std::getenv("EDL_BATCHED_KERNELS");
     bool res = !(e && *e);
-    for (size_t k = 0; k < idx.size() && res; ++k) res = resident_sector(get_sector(c, targets[idx[k]]), sizeof(T));
+    for (size_t k = 0; k < idx.size() && res; ++k)
+      res = resident_sector(get_sector(c, targets[idx[k]]), sizeof(T), idx.size());
     if (res) return tridiag_resident<T>(c, seeds, idx, targets, nlanc, alpha, beta, norm2, nsteps, host_seed);
   }
   std::vector<ChainAlloc<T>> allocs(idx.size());

@@ -30,7 +30,8 @@ struct ResChain {
   double brk_tol;         // relative breakdown threshold on beta
 };
 
-// Whether chains on `s` can run resident: packed hop tables, no non-local
+// Whether chains on `s` can run resident (whether they do: also by size, see the
+// callers): packed hop tables, no non-local
 // block, at most kResMaxRows elements a thread, vector and tables within LDS.
 bool res_ok(const Sector& s, size_t elem);
 // Up to `steps` further Lanczos steps of every chain (device array), one
