@@ -9,7 +9,7 @@
 // What bounds it: one CU's LDS (a hop is a 4-byte table word and an element)
 // and VALU; the chip is filled only by as many chains as CUs.  Position, diagonal
 // and second vector of an element stay in registers: with 8 elements a thread and
-// more in fp64, 12 in fp32, some of them spill (7.6 us a step at 4 900 states, 33
+// more in fp64, 12 in fp32, some of them spill (6.1 us a step at 4 900 states, 32
 // at 15 876), and the callers take the form up to a timed number of states.
 #include <algorithm>
 
