@@ -32,12 +32,14 @@ static size_t on_current_device(F f) {
 }
 
 hipError_t device_malloc_bytes(void** p, size_t bytes) {
-  const hipError_t e = hipMalloc(p, bytes);
+  hipError_t e = hipMalloc(p, bytes);
   if (e != hipErrorOutOfMemory) return e;
   (void)hipGetLastError();
   // (hipFree waits for the device: a cached buffer may have launches queued)
   if (on_current_device([](DevPool& q) { return q.release(); }) == 0) return e;
-  return hipMalloc(p, bytes);
+  e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
 }
 
 size_t device_cached_bytes() {

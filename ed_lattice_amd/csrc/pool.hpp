@@ -12,7 +12,8 @@ namespace edl {
 
 // hipMalloc.  Where the device has no memory left, the cached buffers of every
 // context on it are freed and the allocation is tried once more: memory that no
-// call is using never makes one fail.
+// call is using never makes one fail.  A request that fails for memory leaves no
+// error pending: the launches of the next call look for theirs.
 hipError_t device_malloc_bytes(void** p, size_t bytes);
 template <typename P>
 hipError_t device_malloc(P** p, size_t bytes) {

@@ -132,7 +132,8 @@ CASES = {
   a.give(x);
   void* t = nullptr;
   WANT(device_malloc(&t, 17 * M) == hipErrorOutOfMemory && !t);
-  (void)hipGetLastError();
+  WANT(hipGetLastError() == hipSuccess);
+  WANT(device_malloc(&t, 17 * M) == hipErrorOutOfMemory && hipGetLastError() == hipSuccess);
   WANT(a.cached() == 0 && b.cached() >= 900 * K);
 """,
     # a buffer put back with launches queued and filled again: on the same stream
